@@ -152,6 +152,59 @@ def test_quantize_w4_matches_the_oracle(gpu, dtype, E, N, K, gs):
     assert z.cpu()[0, 2, 0].view(torch.int16).item() == -32768
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+def test_quantize_w4_at_ties_extremes_and_byte_offsets(gpu, dtype, gs):
+    """Columns on a rounding tie (the reference's own division decides), ranges
+    whose reciprocal is subnormal, infinite and NaN weights, a row count that
+    leaves the last workgroup partly empty, and buffers that start at the
+    smallest offset the C entry takes. Exact: bytes and fp16 are a format."""
+    lib_ = load_mod("_lib")
+    N, K = 37, 3 * gs
+    W = 0.02 * torch.randn(N, K, generator=torch.Generator().manual_seed(gs))
+    W[0] = torch.arange(K) % 16                      # scale 1, zero 0: whole numbers
+    W[1] = (torch.arange(K) % 31) / 2                # scale 1: every second column is a tie
+    W[2] = -W[1]                                     # zero 15, ties from below
+    W[3] = (torch.arange(K) % 31) * 0.0078125 + 1.0  # away from 0: clamps
+    W[4, :gs] = 0.0
+    if dtype != torch.float16:
+        W[5] = 1e38 * torch.rand(K, generator=torch.Generator().manual_seed(gs + 1))  # 1 / scale subnormal
+        W[6, :2] = torch.tensor([3e38, -3e38])       # the range overflows
+    W = W.to(dtype)
+    W[7, 5] = float("inf")
+    W[8, gs + 1] = float("nan")                      # takes no part in the range, packs as 0
+    Wn = W.float().numpy()
+    with np.errstate(all="ignore"):
+        g = Wn.reshape(N, 3, gs)
+        mn, mx = np.nanmin(g, -1), np.nanmax(g, -1)
+        sc = (np.maximum(mx - mn, np.float32(1e-8)) / np.float32(15)).astype(np.float32)
+        ze = np.clip(np.round(-mn / sc), 0, 15).astype(np.float32)
+        qq = np.clip(np.round(g / sc[..., None] + ze[..., None]), 0, 15)
+        qq = np.nan_to_num(qq, nan=0.0).astype(np.uint8).reshape(N, K)
+        rs, rz = sc.astype(np.float16), ze.astype(np.float16)
+    rq = qq[:, 0::2] | (qq[:, 1::2] << 4)
+    fin = np.isfinite(Wn).all(-1) & (np.arange(N) != 6)
+    oq, os_, oz = mo.quantize_w4(Wn[fin], gs)
+    assert np.array_equal(oq, rq[fin]) and np.array_equal(os_, rs[fin]) and np.array_equal(oz, rz[fin])
+    for wo, qo in ((0, 0), (2, 0), (0, 1), (2, 3)):  # offsets in elements and bytes
+        wbuf = torch.zeros(N * K + 8, dtype=dtype, device=gpu)
+        wbuf[wo:wo + N * K] = W.reshape(-1).to(gpu)
+        q = torch.full((N * K // 2 + 8,), 0xA5, dtype=torch.uint8, device=gpu)
+        s, z = (torch.empty(N * 3, dtype=torch.float16, device=gpu) for _ in range(2))
+        es = W.element_size()
+        print(f"ksl_quantize_w4 {dtype} gs={gs} offsets {wo} {qo}", flush=True)
+        rc = lib_.load().ksl_quantize_w4(wbuf.data_ptr() + wo * es, lib_.dtype_code(dtype), N, K, gs,
+                                         q.data_ptr() + qo, s.data_ptr(), z.data_ptr(), lib_.stream_of(wbuf))
+        assert rc == 0
+        torch.cuda.synchronize()
+        out = q.cpu().numpy()
+        assert np.array_equal(out[qo:qo + N * K // 2].reshape(N, -1), rq)
+        assert (out[:qo] == 0xA5).all() and (out[qo + N * K // 2:] == 0xA5).all()
+        same = s.cpu().numpy().reshape(N, 3) == rs
+        assert np.array_equal(s.cpu().numpy().view(np.uint16).reshape(N, 3), rs.view(np.uint16)), np.argwhere(~same)
+        assert np.array_equal(z.cpu().numpy().view(np.uint16).reshape(N, 3), rz.view(np.uint16))
+
+
 class _Experts(torch.nn.Module):
     """A bf16 experts module as the model holds it before packing."""
 
