@@ -71,6 +71,65 @@ def test_sampler_vs_oracle(gpu, rows, V, dtype, masked, seed):
     assert torch.equal(s, s2) and torch.equal(a, a2) and torch.equal(h, h2)
 
 
+EDGES = [(V, d) for V in (1, 3, 4, 5, 63, 4095, 4096, 8193, 16384, 16389, 40001) for d in (torch.float32, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("V,dtype", EDGES + [(8193, torch.float16)])
+def test_sampler_at_the_edges_of_a_pass(gpu, V, dtype):
+    """Vocabularies around a lane's 16 columns, a pass and its last units, with
+    16-bit rows that start on every second byte pair, and rows that reach each
+    corner of the draw: even logits (every column is drawn), a decided row, ties,
+    the lowest finite value with and without -inf, infinities and NaN."""
+    ops = load_mod("fused_sampler_ops")
+    rows, seed = 12, 4321
+    low = torch.finfo(dtype).min
+    x = _logits(rows, V, V)
+    x[1] = 0.5                                  # all equal: the noise alone decides, the argmax is 0
+    x[2, V // 2] = 200.0                        # decided
+    x[3] = low
+    x[3, V - 1] = 1.0
+    x[4] = low
+    x[5, ::2] = -float("inf")
+    x[5, V - 1] = 0.0
+    x[6] = torch.arange(V) % 7                  # ties for the maximum
+    x[7] = 1e3 * x[7]                           # scores that round coarsely
+    x[8] = -1e4
+    x[9, 0] = 60.0
+    x[10, V - 1] = 60.0
+    x[11] = x[11].abs() * -1.0
+    x = x.to(dtype)
+    x32 = x.float().numpy()
+    print(f"sampler edges V={V} {dtype}", flush=True)
+    h = ops.fused_entropy(x.to(gpu))
+    s, a, h2 = ops.sample_step(x.to(gpu), seed)
+    s3, a3 = ops.gumbel_argmax_sample(x.to(gpu), seed)
+    y = x.clone().to(gpu)
+    y[0, 0] = float("inf")
+    y[1] = float("nan")
+    y[2] = -float("inf")
+    y[3, V // 3] = float("nan")
+    sy, ay, hy = (t.cpu() for t in ops.sample_step(y, seed))
+    torch.cuda.synchronize()
+    p = torch.softmax(x.double(), -1)
+    ref_h = -(p * torch.where(p > 0, p.log(), torch.zeros_like(p))).sum(-1).numpy()
+    # sums of up to V terms of both signs: a few fp32 ulps of the terms' own size
+    assert np.abs(h.cpu().numpy() - ref_h).max() <= 4e-6 * max(1.0, np.log(V))
+    assert np.abs(h2.cpu().numpy() - ref_h).max() <= 4e-6 * max(1.0, np.log(V))
+    # _check_sample's >= 99% of rows is for hundreds of rows; here near-ties alone may differ
+    ref_s, ref_a, margin = so.gumbel_argmax(x32, seed, fast=True)
+    assert np.array_equal(a.cpu().numpy(), ref_a) and np.array_equal(a3.cpu().numpy(), ref_a)
+    clear = margin > MARGIN
+    assert (s.cpu().numpy() == ref_s)[clear].all() and torch.equal(s, s3)
+    # an infinite logit wins both; nothing is taken of NaN and -inf rows; a single NaN is passed over
+    assert sy[0] == 0 and ay[0] == 0 and torch.isnan(hy[0])
+    assert sy[1] == 0 and ay[1] == 0 and torch.isnan(hy[1])
+    assert sy[2] == 0 and ay[2] == 0 and torch.isnan(hy[2])
+    if V > 1:
+        x32[3, V // 3] = -np.inf
+        ref_s, ref_a, _ = so.gumbel_argmax(x32[3:4], seed + 3, fast=True)
+        assert sy[3] == ref_s[0] and ay[3] == ref_a[0]
+
+
 def test_sampler_strided_rows_and_shapes(gpu):
     ops = load_mod("fused_sampler_ops")
     x = _logits(2 * 12, 3000, 21).reshape(2, 12, 3000)
