@@ -124,10 +124,27 @@ def dtype_code(dt: torch.dtype) -> int:
         raise TypeError(f"unsupported dtype {dt}; expected float32, float16 or bfloat16") from None
 
 
-def stream_of(t: torch.Tensor) -> ctypes.c_void_p:
+# The current stream's handle without building a torch.cuda.Stream for it
+# (0.1 against 1.5 us per call).
+_current_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def raw_stream(t: torch.Tensor) -> int:
+    """The handle of the current stream of t's device, for a ctypes argument."""
     if not t.is_cuda:
         raise ValueError("tensor must be on a GPU (device 'cuda')")
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return _current_raw_stream(t.get_device())
+
+
+def stream_of(t: torch.Tensor) -> ctypes.c_void_p:
+    return ctypes.c_void_p(raw_stream(t))
+
+
+# The hot wrappers write only into tensors they allocate themselves, which never
+# require a gradient, so they need no torch.no_grad() around them (2 us per call).
+def addr(t: torch.Tensor | None) -> int:
+    """t's address for a ctypes pointer argument (the argument types convert it)."""
+    return 0 if t is None else t.data_ptr()
 
 
 def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:

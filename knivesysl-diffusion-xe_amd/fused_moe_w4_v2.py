@@ -384,7 +384,7 @@ def enable_pack(exp, cache: dict | None = None):
 
 def pack_ptrs(exp):
     """(gu_pack, dn_pack) device pointers for the C forwards (NULL without a pack)."""
-    return _lib.ptr(getattr(exp, "gu_pack", None)), _lib.ptr(getattr(exp, "dn_pack", None))
+    return _lib.addr(getattr(exp, "gu_pack", None)), _lib.addr(getattr(exp, "dn_pack", None))
 
 
 def moe_workspace(T: int, tk: int, E: int, H: int, I: int, device) -> torch.Tensor:
@@ -392,7 +392,6 @@ def moe_workspace(T: int, tk: int, E: int, H: int, I: int, device) -> torch.Tens
     return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
 
 
-@torch.no_grad()
 def fused_moe_w4_v2(hidden: torch.Tensor, exp, topk_ids: torch.Tensor, topk_w: torch.Tensor,
                     workspace: torch.Tensor | None = None) -> torch.Tensor:
     T, K = hidden.shape
@@ -425,12 +424,12 @@ def fused_moe_w4_v2(hidden: torch.Tensor, exp, topk_ids: torch.Tensor, topk_w: t
         workspace = moe_workspace(T, tk, E, K, I, dev)
     lib = _lib.load()
     rc = lib.ksl_moe_w4a16_forward(
-        _lib.ptr(hidden), _lib.dtype_code(hidden.dtype), hidden.stride(0),
-        _lib.ptr(ids), _lib.ptr(w), _lib.dtype_code(w.dtype),
-        _lib.ptr(exp.gu_q), _lib.ptr(exp.gu_s), _lib.ptr(exp.gu_z),
-        _lib.ptr(exp.dn_q), _lib.ptr(exp.dn_s), _lib.ptr(exp.dn_z), dn_layout(exp), *pack_ptrs(exp),
+        _lib.addr(hidden), _lib.dtype_code(hidden.dtype), hidden.stride(0),
+        _lib.addr(ids), _lib.addr(w), _lib.dtype_code(w.dtype),
+        _lib.addr(exp.gu_q), _lib.addr(exp.gu_s), _lib.addr(exp.gu_z),
+        _lib.addr(exp.dn_q), _lib.addr(exp.dn_s), _lib.addr(exp.dn_z), dn_layout(exp), *pack_ptrs(exp),
         T, tk, E, K, I, exp._ksl_act,
-        _lib.ptr(y), _lib.dtype_code(y_dtype), y.stride(0),
-        _lib.ptr(workspace), workspace.numel(), _lib.stream_of(hidden))
+        _lib.addr(y), _lib.dtype_code(y_dtype), y.stride(0),
+        _lib.addr(workspace), workspace.numel(), _lib.raw_stream(hidden))
     _lib.check(rc, "ksl_moe_w4a16_forward")
     return y if y_dtype == out_dtype else y.to(out_dtype)

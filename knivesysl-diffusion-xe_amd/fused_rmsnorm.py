@@ -17,14 +17,17 @@ from . import _lib
 
 
 def fused_rmsnorm(x: torch.Tensor, weight: torch.Tensor | None, eps: float) -> torch.Tensor:
+    # At a few hundred rows the launch costs more host time than the kernel runs:
+    # whatever is already a contiguous matrix or vector goes in as it is.
     orig = x.shape
-    x2 = x.reshape(-1, orig[-1]).contiguous()
+    flat = len(orig) == 2 and orig[1] > 0
+    x2 = x if flat and x.is_contiguous() else x.reshape(-1, orig[-1]).contiguous()
     rows, n_cols = x2.shape
     y = torch.empty_like(x2)
     if weight is not None:
         if weight.device != x.device:
             raise ValueError("weight must be on the same device as x")
-        w = weight.reshape(-1).contiguous()
+        w = weight if weight.dim() == 1 and weight.is_contiguous() else weight.reshape(-1).contiguous()
         if w.numel() != n_cols:
             raise ValueError(f"weight has {w.numel()} elements, expected {n_cols}")
         wcode = _lib.dtype_code(w.dtype)
@@ -32,12 +35,12 @@ def fused_rmsnorm(x: torch.Tensor, weight: torch.Tensor | None, eps: float) -> t
         w = None
         wcode = _lib.DTYPE_BF16
     xcode = _lib.dtype_code(x2.dtype)
-    lib = _lib.load()
-    rc = lib.ksl_rmsnorm(_lib.ptr(x2), xcode, _lib.ptr(w), wcode, _lib.ptr(y), xcode,
-                         rows, n_cols, x2.stride(0) if rows else n_cols, y.stride(0) if rows else n_cols,
-                         float(eps), _lib.stream_of(x2))
-    _lib.check(rc, "ksl_rmsnorm")
-    return y.reshape(orig)
+    rc = _lib.load().ksl_rmsnorm(x2.data_ptr(), xcode, _lib.addr(w), wcode, y.data_ptr(), xcode,
+                                 rows, n_cols, x2.stride(0) if rows else n_cols, y.stride(0) if rows else n_cols,
+                                 float(eps), _lib.raw_stream(x2))
+    if rc:
+        _lib.check(rc, "ksl_rmsnorm")
+    return y if flat else y.reshape(orig)
 
 
 def _fused_forward(self, x):

@@ -26,19 +26,17 @@ def _rows(logits: torch.Tensor) -> torch.Tensor:
     return x
 
 
-@torch.no_grad()
 def fused_entropy(logits: torch.Tensor) -> torch.Tensor:
     """logits [..., V] -> entropy [...] fp32 (nats), one pass."""
     x = _rows(logits)
     rows, V = x.shape
     h = torch.empty(rows, dtype=torch.float32, device=x.device)
-    rc = _lib.load().ksl_entropy(_lib.ptr(x), _lib.dtype_code(x.dtype), rows, V, x.stride(0) if rows else V,
-                                 _lib.ptr(h), _lib.stream_of(x))
+    rc = _lib.load().ksl_entropy(_lib.addr(x), _lib.dtype_code(x.dtype), rows, V, x.stride(0) if rows else V,
+                                 _lib.addr(h), _lib.raw_stream(x))
     _lib.check(rc, "ksl_entropy")
     return h.view(logits.shape[:-1])
 
 
-@torch.no_grad()
 def gumbel_argmax_sample(logits: torch.Tensor, seed: int):
     """logits [..., V] -> (sampled idx, argmax idx) int64 [...]. Gumbel-max ==
     Categorical sample; seed is an integer (the row's generator key is seed + row)."""
@@ -46,14 +44,13 @@ def gumbel_argmax_sample(logits: torch.Tensor, seed: int):
     rows, V = x.shape
     samp = torch.empty(rows, dtype=torch.int64, device=x.device)
     amax = torch.empty(rows, dtype=torch.int64, device=x.device)
-    rc = _lib.load().ksl_gumbel_argmax(_lib.ptr(x), _lib.dtype_code(x.dtype), rows, V,
-                                       x.stride(0) if rows else V, int(seed), _lib.ptr(samp), _lib.ptr(amax),
-                                       _lib.stream_of(x))
+    rc = _lib.load().ksl_gumbel_argmax(_lib.addr(x), _lib.dtype_code(x.dtype), rows, V,
+                                       x.stride(0) if rows else V, int(seed), _lib.addr(samp), _lib.addr(amax),
+                                       _lib.raw_stream(x))
     _lib.check(rc, "ksl_gumbel_argmax")
     return samp.view(logits.shape[:-1]), amax.view(logits.shape[:-1])
 
 
-@torch.no_grad()
 def sample_step(logits: torch.Tensor, seed: int):
     """gumbel_argmax_sample and fused_entropy from one read of the logits:
     (sampled, argmax, entropy)."""
@@ -62,8 +59,8 @@ def sample_step(logits: torch.Tensor, seed: int):
     samp = torch.empty(rows, dtype=torch.int64, device=x.device)
     amax = torch.empty(rows, dtype=torch.int64, device=x.device)
     h = torch.empty(rows, dtype=torch.float32, device=x.device)
-    rc = _lib.load().ksl_sample_step(_lib.ptr(x), _lib.dtype_code(x.dtype), rows, V, x.stride(0) if rows else V,
-                                     int(seed), _lib.ptr(samp), _lib.ptr(amax), _lib.ptr(h), _lib.stream_of(x))
+    rc = _lib.load().ksl_sample_step(_lib.addr(x), _lib.dtype_code(x.dtype), rows, V, x.stride(0) if rows else V,
+                                     int(seed), _lib.addr(samp), _lib.addr(amax), _lib.addr(h), _lib.raw_stream(x))
     _lib.check(rc, "ksl_sample_step")
     shape = logits.shape[:-1]
     return samp.view(shape), amax.view(shape), h.view(shape)

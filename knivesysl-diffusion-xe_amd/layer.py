@@ -42,7 +42,6 @@ def _prepare(exp, x, E, H, I):
     return x
 
 
-@torch.no_grad()
 def moe_layer(x: torch.Tensor, norm_w: torch.Tensor | None, eps: float, exp, topk_ids: torch.Tensor,
               topk_w: torch.Tensor, workspace: torch.Tensor | None = None) -> torch.Tensor:
     T, H = x.shape
@@ -63,13 +62,13 @@ def moe_layer(x: torch.Tensor, norm_w: torch.Tensor | None, eps: float, exp, top
     if workspace is None:
         workspace = moe_workspace(T, tk, E, H, I, x.device)
     rc = _lib.load().ksl_moe_layer_forward(
-        _lib.ptr(x), _lib.dtype_code(x.dtype), x.stride(0), _lib.ptr(nw),
+        _lib.addr(x), _lib.dtype_code(x.dtype), x.stride(0), _lib.addr(nw),
         _lib.dtype_code(nw.dtype) if nw is not None else _lib.DTYPE_BF16, float(eps),
-        _lib.ptr(ids), _lib.ptr(w), _lib.dtype_code(w.dtype),
-        _lib.ptr(exp.gu_q), _lib.ptr(exp.gu_s), _lib.ptr(exp.gu_z),
-        _lib.ptr(exp.dn_q), _lib.ptr(exp.dn_s), _lib.ptr(exp.dn_z), dn_layout(exp), *pack_ptrs(exp),
-        T, tk, E, H, I, exp._ksl_act, _lib.ptr(y), _lib.dtype_code(y.dtype), y.stride(0),
-        _lib.ptr(workspace), workspace.numel(), _lib.stream_of(x))
+        _lib.addr(ids), _lib.addr(w), _lib.dtype_code(w.dtype),
+        _lib.addr(exp.gu_q), _lib.addr(exp.gu_s), _lib.addr(exp.gu_z),
+        _lib.addr(exp.dn_q), _lib.addr(exp.dn_s), _lib.addr(exp.dn_z), dn_layout(exp), *pack_ptrs(exp),
+        T, tk, E, H, I, exp._ksl_act, _lib.addr(y), _lib.dtype_code(y.dtype), y.stride(0),
+        _lib.addr(workspace), workspace.numel(), _lib.raw_stream(x))
     _lib.check(rc, "ksl_moe_layer_forward")
     return y
 

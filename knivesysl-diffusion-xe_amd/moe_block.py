@@ -87,14 +87,14 @@ def moe_block_forward(layer, residual: torch.Tensor, hidden_states_1: torch.Tens
         return y.reshape(residual.shape)
     ws = moe_workspace(T, tk, E, H, I, dev)
     rc = _lib.load().ksl_moe_block_forward(
-        _lib.ptr(x), x.stride(0), _lib.ptr(pre_w), float(pre.eps),
-        _lib.ptr(ids), _lib.ptr(w), _lib.dtype_code(w.dtype),
-        _lib.ptr(exp.gu_q), _lib.ptr(exp.gu_s), _lib.ptr(exp.gu_z),
-        _lib.ptr(exp.dn_q), _lib.ptr(exp.dn_s), _lib.ptr(exp.dn_z), dn_layout(exp), *pack_ptrs(exp),
+        _lib.addr(x), x.stride(0), _lib.addr(pre_w), float(pre.eps),
+        _lib.addr(ids), _lib.addr(w), _lib.dtype_code(w.dtype),
+        _lib.addr(exp.gu_q), _lib.addr(exp.gu_s), _lib.addr(exp.gu_z),
+        _lib.addr(exp.dn_q), _lib.addr(exp.dn_s), _lib.addr(exp.dn_z), dn_layout(exp), *pack_ptrs(exp),
         T, tk, E, H, I, exp._ksl_act,
-        _lib.ptr(h1), h1.stride(0), _lib.ptr(post2_w), float(post2.eps), _lib.ptr(post_w), float(post.eps),
-        _lib.ptr(ls), _lib.DTYPE_BF16 if ls is None else _lib.dtype_code(ls.dtype),
-        _lib.ptr(y), y.stride(0), _lib.ptr(ws), ws.numel(), _lib.stream_of(x))
+        _lib.addr(h1), h1.stride(0), _lib.addr(post2_w), float(post2.eps), _lib.addr(post_w), float(post.eps),
+        _lib.addr(ls), _lib.DTYPE_BF16 if ls is None else _lib.dtype_code(ls.dtype),
+        _lib.addr(y), y.stride(0), _lib.addr(ws), ws.numel(), _lib.raw_stream(x))
     _lib.check(rc, "ksl_moe_block_forward")
     return y.reshape(residual.shape)
 

@@ -14,11 +14,10 @@ import torch
 from . import _lib
 
 
-@torch.no_grad()
 def router_forward(self, hidden_states: torch.Tensor):
     """(router_probabilities fp32 [T, E], top_k_weights fp32 [T, k],
     top_k_index int64 [T, k]) as DiffusionGemmaTextRouter.forward returns them."""
-    x = hidden_states.reshape(-1, hidden_states.shape[-1])
+    x = hidden_states if hidden_states.dim() == 2 else hidden_states.reshape(-1, hidden_states.shape[-1])
     if x.stride(-1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         x = x.clone(memory_format=torch.contiguous_format)  # a fresh, aligned copy
     T, H = x.shape
@@ -29,15 +28,16 @@ def router_forward(self, hidden_states: torch.Tensor):
     for t in (self.scale, proj, self.per_expert_scale):
         if t.dtype != torch.bfloat16 or t.device != x.device:
             raise TypeError("router parameters must be bf16 tensors on the hidden states' device")
-        params.append(t.contiguous())
+        params.append(t if t.is_contiguous() else t.contiguous())
     scale, proj, pes = params
     probs = torch.empty(T, E, dtype=torch.float32, device=x.device)
     topk_w = torch.empty(T, k, dtype=torch.float32, device=x.device)
     topk_ids = torch.empty(T, k, dtype=torch.int64, device=x.device)
-    rc = _lib.load().ksl_moe_router(_lib.ptr(x), _lib.dtype_code(x.dtype), x.stride(0), _lib.ptr(scale),
-                                    _lib.ptr(proj), _lib.ptr(pes), _lib.DTYPE_BF16, float(self.eps), T, H, E, k,
-                                    _lib.ptr(probs), _lib.ptr(topk_w), _lib.ptr(topk_ids), _lib.stream_of(x))
-    _lib.check(rc, "ksl_moe_router")
+    rc = _lib.load().ksl_moe_router(x.data_ptr(), _lib.dtype_code(x.dtype), x.stride(0), scale.data_ptr(),
+                                    proj.data_ptr(), pes.data_ptr(), _lib.DTYPE_BF16, float(self.eps), T, H, E, k,
+                                    probs.data_ptr(), topk_w.data_ptr(), topk_ids.data_ptr(), _lib.raw_stream(x))
+    if rc:
+        _lib.check(rc, "ksl_moe_router")
     return probs, topk_w, topk_ids
 
 

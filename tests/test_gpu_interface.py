@@ -259,3 +259,36 @@ def test_repack_cache_binds_only_a_modules_own_weights(gpu):
     y_b = v2.fused_moe_w4_v2(hidden, b, idsg, wg)
     torch.cuda.synchronize()
     assert torch.equal(y_b.view(torch.int16), y_ref.view(torch.int16))
+
+
+def test_wrappers_take_tensors_that_require_a_gradient(gpu):
+    """In grad mode, with inputs that require a gradient or are views, the
+    wrappers give the same results as without, and outputs that require none;
+    each launches on the current stream."""
+    norm, router = load_mod("fused_rmsnorm"), load_mod("router")
+    layer, wl, ops = load_mod("layer"), load_mod("workloads"), load_mod("fused_sampler_ops")
+    T, H, E, I, k = 37, 256, 16, 128, 4
+    x, nw, ids, w = (t.to(gpu) for t in wl.layer_inputs(T, 7, E=E, k=k, H=H))
+    exp = wl.make_experts(E, H, I, 7, act="silu").to(gpu)
+    rt = torch.nn.Module()
+    rt.scale, rt.per_expert_scale, rt.eps = nw.clone(), torch.ones(E, dtype=torch.bfloat16, device=gpu), 1e-6
+    rt.proj = torch.nn.Linear(H, E, bias=False, dtype=torch.bfloat16, device=gpu)
+    rt.config = type("Config", (), {"top_k_experts": k})
+
+    def calls(x, nw, w):
+        y = [norm.fused_rmsnorm(x, nw, 1e-6), norm.fused_rmsnorm(x[None, ::2], nw, 1e-6),
+             layer.moe_layer(x, nw, 1e-6, exp, ids, w), layer.moe_layer(x[1:, :], nw, 1e-6, exp, ids[1:], w[1:]),
+             ops.fused_entropy(x.float())]
+        return y + list(router.router_forward(rt, x)) + list(ops.sample_step(x.float(), 3))
+
+    with torch.no_grad():
+        want = calls(x, nw, w)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = calls(x.clone().requires_grad_(), torch.nn.Parameter(nw), w.clone().requires_grad_())
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    assert all(not g.requires_grad and torch.equal(a, g) for a, g in zip(want, got))
+    with pytest.raises(ValueError):
+        norm.fused_rmsnorm(torch.zeros(2, 8), None, 1e-6)
