@@ -205,6 +205,13 @@ __device__ __forceinline__ ZeroPair zero_pair(f16 z) {
     return ZeroPair{f16x2{a, a}, f16x2{b, b}};
 }
 
+// Zero-point pairs from a nibble z: (1024 + z) and (64 + z) as fp16 bits
+// (0x6400 | z, 0x5400 | z << 4), both halves of each pair.
+__device__ __forceinline__ ZeroPair zero_pair_nib(uint32_t z) {
+    const uint32_t lo = 0x6400u | z, hi = 0x5400u | (z << 4);
+    return ZeroPair{__builtin_bit_cast(f16x2, lo | (lo << 16)), __builtin_bit_cast(f16x2, hi | (hi << 16))};
+}
+
 __device__ __forceinline__ f16x8 nib8_minus_zero(uint32_t w, const ZeroPair& zc, const NibConsts& k) {
     const uint32_t w8 = w >> 8;
     const f16x2 h0 = __builtin_bit_cast(f16x2, (w & k.m_lo) | k.b_lo) - zc.lo;

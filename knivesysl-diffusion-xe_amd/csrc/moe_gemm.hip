@@ -278,22 +278,25 @@ __device__ __forceinline__ void gateup_produce_1w(const GuArgs& A, int e, int c0
     }
 }
 
+// Scale / zero table of the per-item kernel: [s_gate | z_gate | s_up | z_up], n fp16 each.
+struct GuTab16 {
+    const f16* sz;
+    int n;
+    __device__ __forceinline__ float scale(int j, int i) const { return static_cast<float>(sz[2 * j * n + i]); }
+    __device__ __forceinline__ ZeroPair zero(int j, int i) const { return zero_pair(sz[(2 * j + 1) * n + i]); }
+};
+
 // One quantisation group g of a consumer wave: its gate and up weight words in
 // slot sp, decoded against their zero-points, times the MT activation tiles
-// of the slot; the fp32 group partials are scaled into acc. sz: the
-// [s_gate | z_gate | s_up | z_up] table of the workgroup's rows, kCols x G each.
-template <int NC, int MT>
-__device__ __forceinline__ void gateup_group(const char* __restrict__ sp, const f16* __restrict__ sz, int G, int g,
+// of the slot; the fp32 group partials are scaled into acc. tab: the scales and
+// zero-points of the workgroup's kCols gate (j = 0) and up (j = 1) rows, G each.
+template <int NC, int MT, typename Tab>
+__device__ __forceinline__ void gateup_group(const char* __restrict__ sp, const Tab& tab, int G, int g,
                                              const NibConsts& kn, f32x4 (&acc)[2][MT]) {
     constexpr int kSlotW = 2 * NC * kBlk;
-    constexpr int kc = 16 * NC;
     const int wave = wave_id();
     const int lane = threadIdx.x & (kWave - 1);
     const int col = lane & 15, c = lane >> 4;
-    const f16* s_g = sz;
-    const f16* z_g = sz + kc * G;
-    const f16* s_u = sz + 2 * kc * G;
-    const f16* z_u = sz + 3 * kc * G;
     const int r = wave * 16 + col;  // row of the tile within the workgroup
     const int fo = frag_pos(col, c) * 16;
     f32x4 part[2][MT];
@@ -306,7 +309,7 @@ __device__ __forceinline__ void gateup_group(const char* __restrict__ sp, const 
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         wv[j] = *reinterpret_cast<const u32x4*>(sp + (wave * 2 + j) * kBlk + fo);
-        zc[j] = zero_pair((j ? z_u : z_g)[r * G + g]);
+        zc[j] = tab.zero(j, r * G + g);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -322,7 +325,7 @@ __device__ __forceinline__ void gateup_group(const char* __restrict__ sp, const 
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const float sc = static_cast<float>((j ? s_u : s_g)[r * G + g]);
+        const float sc = tab.scale(j, r * G + g);
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -382,7 +385,7 @@ __device__ __forceinline__ void gateup_consume(const GuArgs& A, int c0, const ch
     __syncthreads();  // group 0 and the scale table are ready
     int slot = 0;
     for (int g = 0; g < G; ++g) {
-        gateup_group<NC, MT>(lds + slot * S::kSlot, lds_sz, G, g, kn, acc);
+        gateup_group<NC, MT>(lds + slot * S::kSlot, GuTab16{lds_sz, S::kCols * G}, G, g, kn, acc);
         slot = slot + 1 == R ? 0 : slot + 1;
         __syncthreads();
     }
@@ -481,6 +484,13 @@ __global__ __launch_bounds__((NC + NP) * kWave) void gateup_act_kernel(GuArgs A)
 // first item gets a light second one. The column blocks of a matched expert
 // follow those of its partner, so they stay together on one XCD.
 // Arithmetic and outputs are those of gateup_act_kernel, bit for bit.
+//
+// Wide form: with 33 to 64 rows per expert (a prompt of a page) a 32-row pass
+// streams the item's weights from L2 and decodes them a second time, and the
+// launch took 100 us instead of a canvas's 55. Passes of 64 rows (four M tiles
+// against one decoded fragment) take 1.2 us per group instead of twice 1.0; the
+// ring's slots grow to 38 KB, and the zero-points are kept as nibbles so that
+// two tables still fit (155 KB at H = 2816).
 constexpr int kFlowMaxItems = 64;  // items per workgroup (table entries)
 constexpr int kFlowR = 3;          // ring depth
 constexpr int kFlowMinG = 8;       // groups per pass: the next pass's token ids go
@@ -491,14 +501,32 @@ constexpr int kFlowMinG = 8;       // groups per pass: the next pass's token ids
 using ConstI32 = const int32_t __attribute__((address_space(4)));
 __device__ __forceinline__ const ConstI32* as_scalar_i32(const int32_t* p) { return (const ConstI32*)p; }
 
-template <int NC>
+// Table of the wide form: [s_gate | s_up] fp16, then [z_gate | z_up] as nibbles
+// (element i in byte i / 2, low nibble first), n elements each.
+struct GuTabNib {
+    const f16* s;
+    int n;
+    __device__ __forceinline__ float scale(int j, int i) const { return static_cast<float>(s[j * n + i]); }
+    __device__ __forceinline__ ZeroPair zero(int j, int i) const {
+        const uint8_t* z = reinterpret_cast<const uint8_t*>(s + 2 * n) + j * (n / 2);
+        return zero_pair_nib((static_cast<uint32_t>(z[i >> 1]) >> ((i & 1) * 4)) & 15u);
+    }
+};
+
+// MTX: M tiles per pass, 2 or (the wide form) 4.
+template <int NC, int MTX>
 struct GuFlowShape {
     using B = GuShape<NC, 1, kFlowR>;
-    static constexpr size_t sz_bytes(int G) { return static_cast<size_t>(4) * B::kCols * G * 2; }
-    static constexpr size_t sz_off(int G, int buf) { return static_cast<size_t>(kFlowR) * B::kSlot + buf * sz_bytes(G); }
+    using Tab = std::conditional_t<MTX == 2, GuTab16, GuTabNib>;
+    static constexpr int kPass = 16 * MTX;                       // rows per pass
+    static constexpr int kSlot = B::kSlotW + 4 * MTX * kBlk;
+    static constexpr size_t sz_bytes(int G) {
+        return MTX == 2 ? static_cast<size_t>(4) * B::kCols * G * 2 : static_cast<size_t>(5) * B::kCols * G;
+    }
+    static constexpr size_t sz_off(int G, int buf) { return static_cast<size_t>(kFlowR) * kSlot + buf * sz_bytes(G); }
     static constexpr size_t tok_off(int G) { return sz_off(G, 2); }
     // item table: (first sorted slot, rows, expert, first column) per item
-    static constexpr size_t info_off(int G) { return tok_off(G) + 2 * 16 * kMaxMt * 4; }
+    static constexpr size_t info_off(int G) { return tok_off(G) + 2 * kPass * 4; }
     static constexpr size_t lds_bytes(int G) { return info_off(G) + kFlowMaxItems * 16; }
 };
 
@@ -577,9 +605,10 @@ __device__ __forceinline__ GuPass gu_flow_seek(int k, int m0, int K, const int4&
     return GuPass{K, 0, 0, 0};
 }
 
+template <int kPass>
 __device__ __forceinline__ int gu_flow_npass(int K, const int4& tab) {
     int n = 0;
-    for (int k = 0; k < K; ++k) n += (__builtin_amdgcn_readlane(tab.y, k) + 16 * kMaxMt - 1) / (16 * kMaxMt);
+    for (int k = 0; k < K; ++k) n += (__builtin_amdgcn_readlane(tab.y, k) + kPass - 1) / kPass;
     return n;
 }
 
@@ -588,41 +617,56 @@ __device__ __forceinline__ void gu_flow_item(const int4& tab, int k, int& e, int
     c0 = __builtin_amdgcn_readlane(tab.w, k);
 }
 
-// The scale / zero table of an item's kCols rows: four [kCols x G] fp16 blocks
-// (s_gate, z_gate, s_up, z_up), each contiguous in global memory, fetched by
-// the consumer threads into registers (issue) and written to LDS (commit).
-template <int NC>
+// The scale / zero table of an item's kCols gate and kCols up rows: 16-byte
+// chunks of the scales and of the zero-points at the same place (contiguous in
+// global memory per half: the gate rows, then the up rows), fetched by the
+// consumer threads into registers (issue) and written to LDS (commit). One
+// 32-bit offset per chunk pair: with a pointer per chunk the wide form's
+// addresses were spilled, and each reload was waited for inside the ring.
+template <int NC, int MTX>
 struct GuSzFetch {
     using S = GuShape<NC, 1, kFlowR>;
-    u32x4 v[S::kSzPer];
-    // chunk k of this thread: 16 bytes of block b at o, or none
-    __device__ __forceinline__ static const u32x4* src(const GuArgs& A, int e, int c0, int G, int k) {
-        const int nq = S::kCols * G * 2 / 16;  // 16-byte chunks per block
-        int i = threadIdx.x + k * NC * kWave;
-        if (i >= 4 * nq) i = 0;  // clamped, never stored
-        const int64_t gate0 = static_cast<int64_t>(e) * 2 * A.I + c0;
-        const int b = i / nq, o = i - b * nq;
-        const f16* base = ((b & 1) ? A.gu_z : A.gu_s) + ((b & 2) ? gate0 + A.I : gate0) * G;
-        return reinterpret_cast<const u32x4*>(base) + o;
-    }
+    static constexpr int kPer = S::kSzPer / 2;  // chunk pairs per thread
+    u32x4 s[kPer], z[kPer];
     __device__ __forceinline__ void issue(const GuArgs& A, int e, int c0, int G) {
+        const int nq = S::kCols * G / 8;  // chunks per half
+        const int64_t gate0 = (static_cast<int64_t>(e) * 2 * A.I + c0) * G;
 #pragma unroll
-        for (int k = 0; k < S::kSzPer; ++k) v[k] = *src(A, e, c0, G, k);
+        for (int k = 0; k < kPer; ++k) {
+            int i = threadIdx.x + k * NC * kWave;
+            if (i >= 2 * nq) i = 0;  // clamped, never stored
+            const uint32_t off = static_cast<uint32_t>(i < nq ? i * 8 : A.I * G + (i - nq) * 8);
+            s[k] = *reinterpret_cast<const u32x4*>(A.gu_s + gate0 + off);
+            z[k] = *reinterpret_cast<const u32x4*>(A.gu_z + gate0 + off);
+        }
     }
     __device__ __forceinline__ void commit(f16* __restrict__ dst, int G) const {
-        const int nq = S::kCols * G * 2 / 16;
+        const int nq = S::kCols * G / 8;
+        u32x4* d = reinterpret_cast<u32x4*>(dst);
 #pragma unroll
-        for (int k = 0; k < S::kSzPer; ++k) {
+        for (int k = 0; k < kPer; ++k) {
             const int i = threadIdx.x + k * NC * kWave;
-            if (i < 4 * nq) reinterpret_cast<u32x4*>(dst)[i] = v[k];
+            if (i >= 2 * nq) continue;
+            if constexpr (MTX == 2) {
+                const int o = i < nq ? i : i + nq;  // [s_gate | z_gate | s_up | z_up]
+                d[o] = s[k];
+                d[o + nq] = z[k];
+            } else {
+                const f16x8 v = __builtin_bit_cast(f16x8, z[k]);
+                uint32_t n = 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) n |= (static_cast<uint32_t>(static_cast<float>(v[j])) & 15u) << (4 * j);
+                d[i] = s[k];
+                reinterpret_cast<uint32_t*>(d + 2 * nq)[i] = n;
+            }
         }
     }
 };
 
-template <int NC>
+template <int NC, int MTX>
 __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restrict__ lds, int w, int items, int K) {
     using S = GuShape<NC, 1, kFlowR>;
-    using F = GuFlowShape<NC>;
+    using F = GuFlowShape<NC, MTX>;
     constexpr int R = kFlowR;
     const int lane = threadIdx.x & (kWave - 1);
     const int rr = lane >> 2, ch = (lane & 3) ^ frag_swz(rr);
@@ -636,7 +680,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
     // the issue cursor's pass: weights of its item (first gate row + the lane's
     // piece), the lane's activation row of each M tile, its M tiles
     const char* wbase = nullptr;
-    int64_t aoff[kMaxMt];
+    int64_t aoff[MTX];
     int mt = 1;
     auto set_item = [&](int e, int c0) {
         wbase = reinterpret_cast<const char*>(A.gu_q) + (static_cast<int64_t>(e) * 2 * A.I + c0) * rowbytes + wlane;
@@ -645,25 +689,25 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
     // repeat it: loaded, never stored): from the consumers' LDS copy (toks)
     // for all passes but a workgroup's first
     auto set_rows = [&](const GuPass& p, const int* toks) {
-        const int mrows = min(p.M - p.m0, 16 * kMaxMt);
-        mt = mrows > 16 ? 2 : 1;
+        const int mrows = min(p.M - p.m0, F::kPass);
+        mt = (mrows + 15) >> 4;
 #pragma unroll
-        for (int t = 0; t < kMaxMt; ++t) aoff[t] = (static_cast<int64_t>(toks[t * 16 + rr]) * A.H + ch * 8) * 2;
+        for (int t = 0; t < MTX; ++t) aoff[t] = (static_cast<int64_t>(toks[t * 16 + rr]) * A.H + ch * 8) * 2;
     };
     // ... and for the first pass from the routing itself, by scalar loads: a
     // vector load here would wait (in-order vmcnt) for the weight groups
     // already in flight
     auto set_rows_first = [&](const GuPass& p) {
-        const int mrows = min(p.M - p.m0, 16 * kMaxMt);
-        mt = mrows > 16 ? 2 : 1;
+        const int mrows = min(p.M - p.m0, F::kPass);
+        mt = (mrows + 15) >> 4;
         const ConstI32* rows = as_scalar_i32(A.sorted_rows) + p.start + p.m0;
-        int v[16 * kMaxMt];  // all loads first (uniform, in flight together), then a per-lane pick
+        int v[F::kPass];  // all loads first (uniform, in flight together), then a per-lane pick
 #pragma unroll
-        for (int i = 0; i < 16 * kMaxMt; ++i) v[i] = rows[min(i, mrows - 1)];
+        for (int i = 0; i < F::kPass; ++i) v[i] = rows[min(i, mrows - 1)];
 #pragma unroll
-        for (int i = 0; i < 16 * kMaxMt; ++i) asm volatile("" : "+s"(v[i]));  // not folded into a per-lane load
+        for (int i = 0; i < F::kPass; ++i) asm volatile("" : "+s"(v[i]));  // not folded into a per-lane load
 #pragma unroll
-        for (int t = 0; t < kMaxMt; ++t) {
+        for (int t = 0; t < MTX; ++t) {
             int row = v[t * 16];
 #pragma unroll
             for (int i = 1; i < 16; ++i) row = rr == i ? v[t * 16 + i] : row;
@@ -671,7 +715,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
         }
     };
     auto issue_w = [&](int g, int slot) {
-        char* base = lds + slot * S::kSlot;
+        char* base = lds + slot * F::kSlot;
 #pragma unroll
         for (int b = 0; b < 2 * NC; ++b) {
             const int wv = b >> 1, j = b & 1;
@@ -679,9 +723,9 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
         }
     };
     auto issue_a = [&](int g, int slot) {
-        char* base = lds + slot * S::kSlot;
+        char* base = lds + slot * F::kSlot;
 #pragma unroll
-        for (int t = 0; t < kMaxMt; ++t)
+        for (int t = 0; t < MTX; ++t)
             if (t < mt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -712,7 +756,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
     vm_wait<0>();
     dma_barrier();
     const int4 tab = gu_flow_table(info, K);
-    const int S_total = gu_flow_npass(K, tab) * G;  // group steps of all passes
+    const int S_total = gu_flow_npass<F::kPass>(K, tab) * G;  // group steps of all passes
     if (!first_rows && S_total > 0) {
         p = gu_flow_seek(0, 0, K, tab);
         int e, c0;
@@ -735,7 +779,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
         int mt_issued = 0;
         if (issued < S_total) {
             if (ig == G) {  // the issue cursor enters the next pass
-                const GuPass q = gu_flow_seek(p.k, p.m0 + 16 * kMaxMt, K, tab);
+                const GuPass q = gu_flow_seek(p.k, p.m0 + F::kPass, K, tab);
                 if (q.k != p.k) {
                     int e, c0;
                     gu_flow_item(tab, q.k, e, c0);
@@ -744,7 +788,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
                 p = q;
                 ++ipass;
                 ig = 0;
-                set_rows(p, tok + (ipass & 1) * 16 * kMaxMt);
+                set_rows(p, tok + (ipass & 1) * F::kPass);
             }
             issue_w(ig, slot_i);
             issue_a(ig, slot_i);
@@ -759,6 +803,10 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
             vm_wait<2 * NC + 4>();
         else if (mt_issued == 2)
             vm_wait<2 * NC + 8>();
+        else if (MTX == 4 && mt_issued == 3)
+            vm_wait<2 * NC + 12>();
+        else if (MTX == 4 && mt_issued == 4)
+            vm_wait<2 * NC + 16>();
         else
             vm_wait<0>();
         dma_barrier();
@@ -769,30 +817,31 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
 // Consumer side of one pass: G barriers. At group 1 the loads for the next pass
 // go out (the expanded rows of its slots from wave 0; the scale / zero table
 // of its item when it starts a new one), at group G/2 they go to LDS.
-template <int ACT, int NC, int MT>
+template <int ACT, int NC, int MTX, int MT>
 __device__ __forceinline__ void gu_flow_consume_pass(const GuArgs& A, char* __restrict__ lds, int& slot,
                                                      const f16* __restrict__ sz, int c0, int row0, int mrows,
                                                      int nrow0, int nmrows, int* __restrict__ ntok, int ne, int nc0,
                                                      f16* __restrict__ nsz) {
-    using S = GuShape<NC, 1, kFlowR>;
+    using F = GuFlowShape<NC, MTX>;
     const int G = A.H >> 7;
     const int tid = threadIdx.x;
     const NibConsts kn = nib_consts();
+    const typename F::Tab tab{sz, F::B::kCols * G};
     f32x4 acc[2][MT];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    GuSzFetch<NC> nf;
+    GuSzFetch<NC, MTX> nf;
     int row = 0;
     for (int g = 0; g < G; ++g) {
-        gateup_group<NC, MT>(lds + slot * S::kSlot, sz, G, g, kn, acc);
+        gateup_group<NC, MT>(lds + slot * F::kSlot, tab, G, g, kn, acc);
         if (g == 1) {
             // the expanded row only: its token (row / topk) is taken at G/2, once it has landed
-            if (ntok && tid < 16 * kMaxMt) row = A.sorted_rows[nrow0 + min(tid, nmrows - 1)];
+            if (ntok && tid < F::kPass) row = A.sorted_rows[nrow0 + min(tid, nmrows - 1)];
             if (nsz) nf.issue(A, ne, nc0, G);
         } else if (g == G / 2) {
-            if (ntok && tid < 16 * kMaxMt) ntok[tid] = row / A.topk;
+            if (ntok && tid < F::kPass) ntok[tid] = row / A.topk;
             if (nsz) nf.commit(nsz, G);
         }
         slot = slot + 1 == kFlowR ? 0 : slot + 1;
@@ -805,11 +854,11 @@ __device__ __forceinline__ void gu_flow_consume_pass(const GuArgs& A, char* __re
     gateup_store<ACT, MT>(A, acc, c0, row0, mrows);
 }
 
-template <int ACT, int NC>
+template <int ACT, int NC, int MTX>
 __device__ __forceinline__ void gu_flow_consume(const GuArgs& A, char* __restrict__ lds, int w, int W, int items,
                                                 int K, bool pair) {
     using S = GuShape<NC, 1, kFlowR>;
-    using F = GuFlowShape<NC>;
+    using F = GuFlowShape<NC, MTX>;
     const int G = A.H >> 7;
     const int nb = A.I / S::kCols;
     int* tok = reinterpret_cast<int*>(lds + F::tok_off(G));
@@ -821,20 +870,20 @@ __device__ __forceinline__ void gu_flow_consume(const GuArgs& A, char* __restric
     const int t0 = xcd_remap(w, items);
     const int e0 = t0 / nb;
     {
-        GuSzFetch<NC> f;
+        GuSzFetch<NC, MTX> f;
         f.issue(A, e0, (t0 - e0 * nb) * S::kCols, G);
         if (wave_id() == 0) gu_flow_fill_table(A, info, w, W, items, K, nb, S::kCols, pair);
         f.commit(sz0, G);
     }
     __syncthreads();  // first barrier: the table, buffer 0 and the first pass's group 0 are ready
     const int4 tab = gu_flow_table(info, K);
-    const int npass = gu_flow_npass(K, tab);
+    const int npass = gu_flow_npass<F::kPass>(K, tab);
     GuPass p = gu_flow_seek(0, 0, K, tab);
     const bool first_rows = __builtin_amdgcn_readlane(tab.y, 0) > 0;
     if (!first_rows && npass > 0) {  // the first pass is a later item's (one more barrier, as the producer)
         int e, c0;
         gu_flow_item(tab, p.k, e, c0);
-        GuSzFetch<NC> f;
+        GuSzFetch<NC, MTX> f;
         f.issue(A, e, c0, G);
         f.commit(sz0, G);
         __syncthreads();
@@ -842,39 +891,54 @@ __device__ __forceinline__ void gu_flow_consume(const GuArgs& A, char* __restric
     int zb = 0;  // table buffer of the current item
     int slot = 0;
     for (int ip = 0; ip < npass; ++ip) {
-        const GuPass q = gu_flow_seek(p.k, p.m0 + 16 * kMaxMt, K, tab);
+        const GuPass q = gu_flow_seek(p.k, p.m0 + F::kPass, K, tab);
         const bool more = q.k < K, fresh = more && q.k != p.k;
         int e, c0, ne = 0, nc0 = 0;
         gu_flow_item(tab, p.k, e, c0);
         if (fresh) gu_flow_item(tab, q.k, ne, nc0);
         const f16* sz = reinterpret_cast<const f16*>(lds + F::sz_off(G, zb));
-        int* ntok = more ? tok + ((ip + 1) & 1) * 16 * kMaxMt : nullptr;
+        int* ntok = more ? tok + ((ip + 1) & 1) * F::kPass : nullptr;
         f16* nsz = fresh ? reinterpret_cast<f16*>(lds + F::sz_off(G, zb ^ 1)) : nullptr;
-        const int mrows = min(p.M - p.m0, 16 * kMaxMt);
-        const int nrow0 = q.start + q.m0, nmrows = more ? min(q.M - q.m0, 16 * kMaxMt) : 1;
-        if (mrows <= 16)
-            gu_flow_consume_pass<ACT, NC, 1>(A, lds, slot, sz, c0, p.start + p.m0, mrows, nrow0, nmrows, ntok, ne, nc0,
-                                             nsz);
-        else
-            gu_flow_consume_pass<ACT, NC, 2>(A, lds, slot, sz, c0, p.start + p.m0, mrows, nrow0, nmrows, ntok, ne, nc0,
-                                             nsz);
+        const int mrows = min(p.M - p.m0, F::kPass);
+        const int nrow0 = q.start + q.m0, nmrows = more ? min(q.M - q.m0, F::kPass) : 1;
+        auto pass = [&](auto mt_c) {
+            gu_flow_consume_pass<ACT, NC, MTX, decltype(mt_c)::value>(A, lds, slot, sz, c0, p.start + p.m0, mrows,
+                                                                      nrow0, nmrows, ntok, ne, nc0, nsz);
+        };
+        if (mrows <= 16) pass(std::integral_constant<int, 1>{});
+        else if (MTX == 2 || mrows <= 32) pass(std::integral_constant<int, 2>{});
+        else if constexpr (MTX == 4) {
+            if (mrows <= 48) pass(std::integral_constant<int, 3>{});
+            else pass(std::integral_constant<int, 4>{});
+        }
         if (fresh) zb ^= 1;
         p = q;
     }
 }
 
-template <int ACT, int NC>
-__global__ __launch_bounds__((NC + 1) * kWave) void gateup_flow_kernel(GuArgs A, int W, int items, int pair) {
+template <int ACT, int NC, int MTX>
+__device__ __forceinline__ void gu_flow(const GuArgs& A, int W, int items, int pair) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int w = blockIdx.x;
     const int K = (items - w + W - 1) / W;  // items of this workgroup (1 .. kFlowMaxItems)
     if (wave_id() >= NC) {
         // the producer issues first on its SIMD after each barrier
         __builtin_amdgcn_s_setprio(3);
-        gu_flow_produce<NC>(A, lds, w, items, K);
+        gu_flow_produce<NC, MTX>(A, lds, w, items, K);
     } else {
-        gu_flow_consume<ACT, NC>(A, lds, w, W, items, K, pair != 0);
+        gu_flow_consume<ACT, NC, MTX>(A, lds, w, W, items, K, pair != 0);
     }
+}
+
+template <int ACT, int NC>
+__global__ __launch_bounds__((NC + 1) * kWave) void gateup_flow_kernel(GuArgs A, int W, int items, int pair) {
+    gu_flow<ACT, NC, 2>(A, W, items, pair);
+}
+
+// The wide form: passes of up to 64 rows.
+template <int ACT, int NC>
+__global__ __launch_bounds__((NC + 1) * kWave) void gateup_flow_wide_kernel(GuArgs A, int W, int items, int pair) {
+    gu_flow<ACT, NC, 4>(A, W, items, pair);
 }
 
 // Dynamic LDS beyond 64 KB: raise a kernel's limit (called once per kernel).
@@ -929,9 +993,9 @@ int launch_gateup_nc(const GuArgs& A, int64_t E, int64_t nrows, int act, hipStre
     return KSL_OK;
 }
 
-template <int NC>
+template <int NC, int MTX>
 int launch_gateup_flow(const GuArgs& A, int act, int W, int items, hipStream_t st) {
-    using F = GuFlowShape<NC>;
+    using F = GuFlowShape<NC, MTX>;
     constexpr int kThreads = (NC + 1) * kWave;
     const size_t lds = F::lds_bytes(A.H / 128);
     if (lds > kLdsDynMax) return KSL_ERR_SHAPE;
@@ -939,20 +1003,17 @@ int launch_gateup_flow(const GuArgs& A, int act, int W, int items, hipStream_t s
     // first-round items, at most one first-round expert per lane of a wave
     const int nb = A.I / GuShape<NC, 1, kFlowR>::kCols;
     const int pair = items == 2 * W && (W / kXcds) % nb == 0 && (items / kXcds) % nb == 0 && W / nb <= kWave;
-    static const bool attr_set =
-        set_max_lds(reinterpret_cast<const void*>(&gateup_flow_kernel<KSL_ACT_GELU_TANH, NC>)) &&
-        set_max_lds(reinterpret_cast<const void*>(&gateup_flow_kernel<KSL_ACT_SILU, NC>)) &&
-        set_max_lds(reinterpret_cast<const void*>(&gateup_flow_kernel<KSL_ACT_NONE, NC>));
-    (void)attr_set;
-    if (act == KSL_ACT_GELU_TANH)
-        hipLaunchKernelGGL((gateup_flow_kernel<KSL_ACT_GELU_TANH, NC>), dim3(W), dim3(kThreads), lds, st, A, W, items,
-                           pair);
-    else if (act == KSL_ACT_SILU)
-        hipLaunchKernelGGL((gateup_flow_kernel<KSL_ACT_SILU, NC>), dim3(W), dim3(kThreads), lds, st, A, W, items, pair);
-    else if (act == KSL_ACT_NONE)
-        hipLaunchKernelGGL((gateup_flow_kernel<KSL_ACT_NONE, NC>), dim3(W), dim3(kThreads), lds, st, A, W, items, pair);
-    else
-        return KSL_ERR_ARG;
+    auto go = [&](auto act_c) {
+        constexpr int ACT = decltype(act_c)::value;
+        constexpr auto kernel = MTX == 2 ? &gateup_flow_kernel<ACT, NC> : &gateup_flow_wide_kernel<ACT, NC>;
+        static const bool attr_set = set_max_lds(reinterpret_cast<const void*>(kernel));
+        (void)attr_set;
+        hipLaunchKernelGGL(kernel, dim3(W), dim3(kThreads), lds, st, A, W, items, pair);
+    };
+    if (act == KSL_ACT_GELU_TANH) go(std::integral_constant<int, KSL_ACT_GELU_TANH>{});
+    else if (act == KSL_ACT_SILU) go(std::integral_constant<int, KSL_ACT_SILU>{});
+    else if (act == KSL_ACT_NONE) go(std::integral_constant<int, KSL_ACT_NONE>{});
+    else return KSL_ERR_ARG;
     KSL_LAUNCH_CHECK();
     return KSL_OK;
 }
@@ -967,7 +1028,7 @@ int gateup_flow_workgroups(int64_t items, int64_t H, int cus) {
     const int W = cus - cus % kXcds;
     const int G = static_cast<int>(H / 128);
     if (W < kXcds || items <= cus || items > static_cast<int64_t>(W) * kFlowMaxItems) return 0;
-    if (G < kFlowMinG || GuFlowShape<NC>::lds_bytes(G) > kLdsDynMax) return 0;
+    if (G < kFlowMinG || GuFlowShape<NC, 2>::lds_bytes(G) > kLdsDynMax) return 0;
     return W;
 }
 
@@ -1468,7 +1529,18 @@ int launch_gateup(const void* a16, const int32_t* sorted_rows, const int32_t* of
         // flowing across its items
         const int64_t items = E * (I / 176);
         const int W = gateup_flow_workgroups(items, H, device_cus());
-        if (W > 0) return launch_gateup_flow<11>(A, act, W, static_cast<int>(items), st);
+        // 64-row passes from an average of 16 rows per expert: below it hardly
+        // an expert has more than 32 rows and the forms take the same time
+        // (layer of 128 tokens 92.5 against 92.3 us, 256 tokens 99.5 / 99.0),
+        // above it the narrow form streams and decodes weights twice
+        // (384 tokens 130 -> 122 us, 741 tokens 184 -> 157 us)
+        // pass)
+        if (W > 0) {
+            const bool wide =
+                nrows_hint >= 16 * E && GuFlowShape<11, 4>::lds_bytes(static_cast<int>(H / 128)) <= kLdsDynMax;
+            return wide ? launch_gateup_flow<11, 4>(A, act, W, static_cast<int>(items), st)
+                        : launch_gateup_flow<11, 2>(A, act, W, static_cast<int>(items), st);
+        }
         return launch_gateup_nc<11, 1, 3>(A, E, nrows_hint, act, st);
     }
     if (I % 128 == 0) return launch_gateup_nc<8, 4, 4>(A, E, nrows_hint, act, st);

@@ -84,13 +84,6 @@ __device__ __forceinline__ void dma4(const void* src, char* lds_block) {
     __builtin_amdgcn_global_load_lds((gbl_vptr)(const_cast<void*>(src)), (lds_vptr)lds_block, 4, 0, 0);
 }
 
-// Zero-point pairs from a nibble z: (1024 + z) and (64 + z) as fp16 bits
-// (0x6400 | z, 0x5400 | z << 4), both halves of each pair.
-__device__ __forceinline__ ZeroPair zero_pair_nib(uint32_t z) {
-    const uint32_t lo = 0x6400u | z, hi = 0x5400u | (z << 4);
-    return ZeroPair{__builtin_bit_cast(f16x2, lo | (lo << 16)), __builtin_bit_cast(f16x2, hi | (hi << 16))};
-}
-
 template <int KIND, int ACT, int LAYOUT>
 __global__ __launch_bounds__(kRbThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void rb_gemm_kernel(RbArgs A) {
     extern __shared__ __attribute__((aligned(16))) char lds[];

@@ -684,3 +684,42 @@ def test_forward_accepts_a_misaligned_contiguous_hidden(gpu):
     assert off.is_contiguous() and off.data_ptr() % 16 != 0
     y = v2.fused_moe_w4_v2(off, exp, ids.to(gpu), w.to(gpu))
     assert torch.equal(ref.view(torch.int16), y.view(torch.int16))
+
+
+def _rows_per_expert_routing(counts, topk, seed):
+    """ids [T, topk] whose expert e appears counts[e] times (sum a multiple of topk)."""
+    flat = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    flat = flat[torch.randperm(flat.numel(), generator=torch.Generator().manual_seed(seed))]
+    return flat.reshape(-1, topk).contiguous()
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("E,H,I,counts", [
+    # one workgroup per CU over 640 items, 64-row passes: every tile count and its edges, empty and heavy experts
+    (160, 1024, 704, [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 80, 97, 128, 129, 200, 3] + [20] * 140),
+    (128, 2816, 704, [33, 48, 49, 64, 65, 0, 112, 113] + [17] * 119 + [21]),  # balanced pairs
+    (128, 2816, 704, [1500] + [4] * 127),                                     # one expert holds most rows
+])
+def test_rows_do_not_depend_on_the_rows_beside_them(gpu, act, E, H, I, counts):
+    """A token's output in a routing of many rows per expert (64-row passes,
+    down with up to four M tiles, heavy experts cut into chunks) has the bits of
+    the same token routed alone in a small call, where every expert has at most
+    one tile of rows."""
+    wl, v2 = load_mod("workloads"), load_mod("fused_moe_w4_v2")
+    topk = 4
+    counts = list(counts)
+    counts[-1] += -sum(counts) % topk
+    ids = _rows_per_expert_routing(counts, topk, E + H)
+    T = ids.shape[0]
+    assert 16 * E <= T * topk <= 8192 or max(counts) > 1000
+    w = torch.rand(T, topk, generator=torch.Generator().manual_seed(1)) + 0.1
+    exp = wl.make_experts(E, H, I, 11, act=act).to(gpu)
+    v2.enable_tiled_down(exp)
+    x = wl.make_hidden(T, H, 12).to(gpu)
+    ids, w = ids.to(gpu), w.to(gpu)
+    print(f"rows beside: E={E} H={H} I={I} T={T} {act} max {max(counts)}", flush=True)
+    y = v2.fused_moe_w4_v2(x, exp, ids, w)
+    few = torch.randperm(T, generator=torch.Generator().manual_seed(2))[:96].to(gpu)
+    alone = torch.cat([v2.fused_moe_w4_v2(x[p], exp, ids[p], w[p]) for p in few.split(4)])
+    torch.cuda.synchronize()
+    assert torch.equal(y[few].view(torch.int16), alone.view(torch.int16))
