@@ -1228,27 +1228,30 @@ __device__ __forceinline__ void dn_pair_mma(const DnTile<G2, TAIL, LAYOUT>& w0, 
 template <int NT>
 __device__ __forceinline__ void dn_store_pair(const f32x4 (&acc0)[NT], const f32x4 (&acc1)[NT], char* o_lds,
                                               __amdgpu_buffer_rsrc_t out, int H, int colw, bool second, int mrows,
-                                              int lane, int row0) {
+                                              int lane) {
     const int col = lane & 15, c = lane >> 4;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const f16x4 v0{static_cast<f16>(acc0[t][0]), static_cast<f16>(acc0[t][1]), static_cast<f16>(acc0[t][2]),
-                       static_cast<f16>(acc0[t][3])};
-        const f16x4 v1{static_cast<f16>(acc1[t][0]), static_cast<f16>(acc1[t][1]), static_cast<f16>(acc1[t][2]),
-                       static_cast<f16>(acc1[t][3])};
-        char* rowp = o_lds + (t * 16 + col) * kDnOutRow;
-        *reinterpret_cast<f16x4*>(rowp + c * 8) = v0;
-        *reinterpret_cast<f16x4*>(rowp + 32 + c * 8) = v1;
-    }
     // lane (r = lane / 4, part = lane % 4): 16 bytes of row r, columns 8 * part ..
     const int r = lane >> 2, part = lane & 3;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(o_lds + (t * 16 + r) * kDnOutRow + part * 16);
-        const int row = t * 16 + r;  // row0 + row of the chunk; mrows counted from row0
-        const bool ok = row < mrows && (second || part < 2);
-        const uint32_t off = ok ? static_cast<uint32_t>(((row0 + row) * H + colw + 8 * part) * 2) : kDropOffset;
-        __builtin_amdgcn_raw_buffer_store_b128(v, out, off, 0, 0);
+    for (int t0 = 0; t0 < NT; t0 += 2) {  // the staging area holds two M tiles
+#pragma unroll
+        for (int t = t0; t < NT && t < t0 + 2; ++t) {
+            const f16x4 v0{static_cast<f16>(acc0[t][0]), static_cast<f16>(acc0[t][1]), static_cast<f16>(acc0[t][2]),
+                           static_cast<f16>(acc0[t][3])};
+            const f16x4 v1{static_cast<f16>(acc1[t][0]), static_cast<f16>(acc1[t][1]), static_cast<f16>(acc1[t][2]),
+                           static_cast<f16>(acc1[t][3])};
+            char* rowp = o_lds + ((t - t0) * 16 + col) * kDnOutRow;
+            *reinterpret_cast<f16x4*>(rowp + c * 8) = v0;
+            *reinterpret_cast<f16x4*>(rowp + 32 + c * 8) = v1;
+        }
+#pragma unroll
+        for (int t = t0; t < NT && t < t0 + 2; ++t) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(o_lds + ((t - t0) * 16 + r) * kDnOutRow + part * 16);
+            const int row = t * 16 + r;
+            const bool ok = row < mrows && (second || part < 2);
+            const uint32_t off = ok ? static_cast<uint32_t>((row * H + colw + 8 * part) * 2) : kDropOffset;
+            __builtin_amdgcn_raw_buffer_store_b128(v, out, off, 0, 0);
+        }
     }
 }
 
@@ -1275,9 +1278,9 @@ __device__ __forceinline__ void dn_stage_a(const DnArgs& A, char* a_lds, int sta
 // by the other waves of the SIMD rather than by a second register buffer (a
 // second buffer, measured, was not faster: the decode, the MFMAs with their
 // LDS reads and the stores already keep the SIMD busy while a wave waits).
-// The M tiles go in passes of at most two over the same weight registers
-// (accumulators for more would not fit), so a chunk of three or four M tiles
-// decodes its weights twice but streams them once.
+// A chunk's M tiles (up to four) go in one pass, one instance per count: with
+// passes of two, a chunk of three or four decoded its weights twice (layer of
+// 741 tokens, 46 rows per expert: 158 -> 143 us; 170 VGPRs at I = 704).
 template <int G2, bool TAIL, int LAYOUT>
 __global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
     constexpr int MTX = kDnMaxMt;
@@ -1332,9 +1335,7 @@ __global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
         for (int k = 0; k < npw; ++k) {
             if (k > 0) fetch(k);
             const int p = wave + k * kDnWaves;
-            // two straight-line passes, not a loop (a loop kept both tiles'
-            // weights and every pass temporary live at once: spills)
-            auto pass = [&](auto nt_c, int t0) {
+            auto pass = [&](auto nt_c) {
                 constexpr int NT = decltype(nt_c)::value;
                 f32x4 acc0[NT], acc1[NT];
 #pragma unroll
@@ -1342,19 +1343,13 @@ __global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
                     acc0[t] = f32x4{0.f, 0.f, 0.f, 0.f};
                     acc1[t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
-                dn_pair_mma<G2, TAIL, LAYOUT, NT>(x0, x1, acc0, acc1, lds + t0 * 2 * G * kBlk, fo, kn);
-                dn_store_pair<NT>(acc0, acc1, o_lds, out, A.H, col0 + 32 * p, 2 * p + 1 < ntiles, mrows - 16 * t0,
-                                  lane, t0 * 16);
+                dn_pair_mma<G2, TAIL, LAYOUT, NT>(x0, x1, acc0, acc1, lds, fo, kn);
+                dn_store_pair<NT>(acc0, acc1, o_lds, out, A.H, col0 + 32 * p, 2 * p + 1 < ntiles, mrows, lane);
             };
-            // an odd last M tile goes in a one-tile pass (half the MFMAs and
-            // LDS reads of a two-tile pass)
-            if (mt == 1) {
-                pass(std::integral_constant<int, 1>{}, 0);
-            } else {
-                pass(std::integral_constant<int, 2>{}, 0);
-                if (mt == 3) pass(std::integral_constant<int, 1>{}, 2);
-                if (mt == 4) pass(std::integral_constant<int, 2>{}, 2);
-            }
+            if (mt == 1) pass(std::integral_constant<int, 1>{});
+            else if (mt == 2) pass(std::integral_constant<int, 2>{});
+            else if (mt == 3) pass(std::integral_constant<int, 3>{});
+            else pass(std::integral_constant<int, 4>{});
         }
     }
 }
@@ -1533,8 +1528,7 @@ int launch_gateup(const void* a16, const int32_t* sorted_rows, const int32_t* of
         // an expert has more than 32 rows and the forms take the same time
         // (layer of 128 tokens 92.5 against 92.3 us, 256 tokens 99.5 / 99.0),
         // above it the narrow form streams and decodes weights twice
-        // (384 tokens 130 -> 122 us, 741 tokens 184 -> 157 us)
-        // pass)
+        // (layer of 384 tokens 130 -> 122 us, of 741 tokens 184 -> 157 us)
         if (W > 0) {
             const bool wide =
                 nrows_hint >= 16 * E && GuFlowShape<11, 4>::lds_bytes(static_cast<int>(H / 128)) <= kLdsDynMax;
