@@ -88,12 +88,10 @@ template <int KIND, int ACT, int LAYOUT>
 __global__ __launch_bounds__(kRbThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void rb_gemm_kernel(RbArgs A) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     constexpr int kWc = KIND == kRbGateUp ? 32 : 64;  // output columns per wave
-    const int tile = xcd_remap(blockIdx.x, gridDim.x);
-    const int unit = tile / A.ncb;
-    const int cb = tile - unit * A.ncb;
-    int e, start, M;
-    find_row_block(A.offsets, A.E, kRbRows, unit, e, start, M);
+    int e, start, M, cb;
+    find_row_block(A.offsets, A.E, kRbRows, blockIdx.x, A.ncb, e, start, M, cb);
     if (M <= 0) return;  // past the last row block (uniform)
+    cb = __builtin_amdgcn_readfirstlane(cb);
     M = __builtin_amdgcn_readfirstlane(M);
     start = __builtin_amdgcn_readfirstlane(start);
     e = __builtin_amdgcn_readfirstlane(e);
@@ -398,7 +396,7 @@ int rb_launch(const RbArgs& A, int64_t nrows, hipStream_t st) {
     (void)attr;
     // row blocks: at most ceil(nrows / 128) + E of them (one partial block per expert)
     const int64_t units = (nrows + kRbRows - 1) / kRbRows + A.E;
-    const int64_t grid = units * A.ncb;
+    const int64_t grid = (units + kXcds - 1) / kXcds * kXcds * A.ncb;  // the same number of blocks for each XCD
     if (grid >= (int64_t(1) << 31)) return KSL_ERR_SHAPE;
     hipLaunchKernelGGL((rb_gemm_kernel<KIND, ACT, LAYOUT>), dim3(static_cast<unsigned>(grid)), dim3(kRbThreads),
                        rb_lds_bytes(A.Gs), st, A);
