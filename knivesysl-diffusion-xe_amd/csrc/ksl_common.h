@@ -489,6 +489,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
 // tokens at popularity rank^-0.6 370 -> 336 us, 1536 even tokens 377 -> 275, 8192
 // tokens at rank^-1.1 1001 -> 945. Equal runs of the blocks that exist: 357, 273
 // and 980, the heavy experts' full blocks all on a few XCDs.) One workgroup barrier, taken by every wave.
+// SKIP = 1 numbers only an expert's blocks after its first.
+template <int SKIP = 0>
 __device__ __forceinline__ void find_row_block(const int32_t* __restrict__ offsets, int E, int rb, int bid, int ncb,
                                                int& e, int& start, int& M, int& cb) {
     __shared__ int info[4];
@@ -510,7 +512,7 @@ __device__ __forceinline__ void find_row_block(const int32_t* __restrict__ offse
                 o0 = offsets[ex];
                 cnt = offsets[ex + 1] - o0;
             }
-            const int nb = (cnt + rb - 1) / rb;
+            const int nb = (max(cnt - SKIP * rb, 0) + rb - 1) / rb;
             int incl = nb;
 #pragma unroll
             for (int off = 1; off < kWave; off <<= 1) {
@@ -519,7 +521,7 @@ __device__ __forceinline__ void find_row_block(const int32_t* __restrict__ offse
             }
             const int excl = base + incl - nb;
             if (ex < E && blk >= excl && blk < excl + nb) {
-                const int b = blk - excl;
+                const int b = blk - excl + SKIP;
                 info[0] = ex;
                 info[1] = o0 + b * rb;
                 info[2] = cnt - b * rb < rb ? cnt - b * rb : rb;

@@ -519,6 +519,7 @@ struct GuFlowShape {
     using B = GuShape<NC, 1, kFlowR>;
     using Tab = std::conditional_t<MTX == 2, GuTab16, GuTabNib>;
     static constexpr int kPass = 16 * MTX;                       // rows per pass
+    static constexpr int kCap = MTX == 2 ? 0x7fffffff : kPass;   // rows per item
     static constexpr int kSlot = B::kSlotW + 4 * MTX * kBlk;
     static constexpr size_t sz_bytes(int G) {
         return MTX == 2 ? static_cast<size_t>(4) * B::kCols * G * 2 : static_cast<size_t>(5) * B::kCols * G;
@@ -540,15 +541,16 @@ struct GuFlowShape {
 // among the first-round experts (most rows first, ties: lower expert first)
 // picks the second-round expert of rank r (fewest rows first, same ties),
 // column block b. All loads go out before any is used.
+// An item holds at most `cap` rows of its expert (the wide form's first chunk).
 __device__ __forceinline__ void gu_flow_fill_table(const GuArgs& A, int4* __restrict__ info, int w, int W, int items,
-                                                   int K, int nb, int kCols, bool pair) {
+                                                   int K, int nb, int kCols, bool pair, int cap) {
     const int lane = threadIdx.x & (kWave - 1);
     if (!pair) {
         if (lane < K) {
             const int tile = xcd_remap(w + lane * W, items);
             const int e = tile / nb;
             const int start = A.offsets[e];
-            info[lane] = int4{start, A.offsets[e + 1] - start, e, (tile - e * nb) * kCols};
+            info[lane] = int4{start, min(A.offsets[e + 1] - start, cap), e, (tile - e * nb) * kCols};
         }
         return;
     }
@@ -560,8 +562,8 @@ __device__ __forceinline__ void gu_flow_fill_table(const GuArgs& A, int4* __rest
         e2 = xcd_remap(wj + W, items) / nb;
         s1 = A.offsets[e1];
         s2 = A.offsets[e2];
-        m1 = A.offsets[e1 + 1] - s1;
-        m2 = A.offsets[e2 + 1] - s2;
+        m1 = min(A.offsets[e1 + 1] - s1, cap);
+        m2 = min(A.offsets[e2 + 1] - s2, cap);
     }
     const int q = w >> 3;
     const int b = q % nb;
@@ -581,6 +583,53 @@ __device__ __forceinline__ void gu_flow_fill_table(const GuArgs& A, int4* __rest
     if (lane == 1) info[1] = second;
 }
 
+// The wide form's further items: every 64-row chunk of an expert after its
+// first, numbered expert by expert, goes round the XCDs (chunk u on XCD u % 8
+// with its nb column blocks), and on an XCD round its W / 8 workgroups. The
+// calling wave appends those of workgroup w to the K items of the table and
+// leaves the number of all in the table's last entry. With the chunks of an
+// expert in one workgroup the launch took as long as the heaviest expert.
+__device__ __forceinline__ void gu_flow_add_chunks(const GuArgs& A, int4* __restrict__ info, int w, int W, int E,
+                                                   int K, int nb, int kCols, int cap) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int per = W / kXcds;
+    int q = w / kXcds;  // this workgroup's places on its XCD: w / 8, + per, + 2 per, ...
+    int n = K, base = 0;
+    for (int e0 = 0; e0 < E; e0 += 2 * kWave) {
+        int st[2], cnt[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {  // both batches' loads go out together
+            const int ex = min(e0 + b * kWave + lane, E - 1);
+            st[b] = A.offsets[ex];
+            cnt[b] = A.offsets[ex + 1];
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int ex = e0 + b * kWave + lane;
+            cnt[b] = ex < E ? cnt[b] - st[b] : 0;
+            const int nch = cap == 64 ? (max(cnt[b] - 64, 0) + 63) >> 6 : 0;
+            if (__ballot(nch > 0) == 0) continue;
+            int incl = nch;
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) {
+                const int o = __shfl_up(incl, off, kWave);
+                if (lane >= off) incl += o;
+            }
+            const int excl = base + incl - nch, end = base + __builtin_amdgcn_readlane(incl, kWave - 1);
+            for (int u = q / nb * kXcds + w % kXcds; u < end; u = q / nb * kXcds + w % kXcds) {
+                if (u >= excl && u < excl + nch) {  // one lane
+                    const int m0 = (u - excl + 1) * 64;
+                    info[n] = int4{st[b] + m0, min(cnt[b] - m0, 64), ex, q % nb * kCols};
+                }
+                ++n;
+                q += per;
+            }
+            base = end;
+        }
+    }
+    if (lane == 0) info[kFlowMaxItems - 1] = int4{n, 0, 0, 0};
+}
+
 // A pass: rows start + m0 .. start + min(M, m0 + 32) - 1 of item k (k == K: none left).
 struct GuPass {
     int k, m0, start, M;
@@ -589,9 +638,17 @@ struct GuPass {
 // The item table held in registers after the first barrier: lane k holds
 // item k (one LDS read per wave); entries are then taken with v_readlane,
 // without LDS round trips at the pass changes.
-__device__ __forceinline__ int4 gu_flow_table(const int4* info, int K) {
+// The wide form's last entry says how many items there are.
+template <int MTX>
+__device__ __forceinline__ int4 gu_flow_table(const int4* info, int& K) {
     const int lane = threadIdx.x & (kWave - 1);
-    return lane < K ? info[lane] : int4{0, 0, 0, 0};
+    if constexpr (MTX == 4) {
+        const int4 t = info[lane];  // entries past the last item are never looked at
+        K = __builtin_amdgcn_readlane(t.x, kFlowMaxItems - 1);
+        return t;
+    } else {
+        return lane < K ? info[lane] : int4{0, 0, 0, 0};
+    }
 }
 
 // The first pass at or after (k, m0) with rows. All values wave-uniform.
@@ -680,7 +737,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
     // the issue cursor's pass: weights of its item (first gate row + the lane's
     // piece), the lane's activation row of each M tile, its M tiles
     const char* wbase = nullptr;
-    int64_t aoff[MTX];
+    int64_t aoff[MTX] = {};
     int mt = 1;
     auto set_item = [&](int e, int c0) {
         wbase = reinterpret_cast<const char*>(A.gu_q) + (static_cast<int64_t>(e) * 2 * A.I + c0) * rowbytes + wlane;
@@ -701,17 +758,21 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
         const int mrows = min(p.M - p.m0, F::kPass);
         mt = (mrows + 15) >> 4;
         const ConstI32* rows = as_scalar_i32(A.sorted_rows) + p.start + p.m0;
-        int v[F::kPass];  // all loads first (uniform, in flight together), then a per-lane pick
 #pragma unroll
-        for (int i = 0; i < F::kPass; ++i) v[i] = rows[min(i, mrows - 1)];
+        for (int h = 0; h < MTX; h += 2) {  // two tiles at a time, as far as there are rows
+            if (h > 0 && mrows <= 16 * h) break;
+            int v[32];  // all loads first (uniform, in flight together), then a per-lane pick
 #pragma unroll
-        for (int i = 0; i < F::kPass; ++i) asm volatile("" : "+s"(v[i]));  // not folded into a per-lane load
+            for (int i = 0; i < 32; ++i) v[i] = rows[min(16 * h + i, mrows - 1)];
 #pragma unroll
-        for (int t = 0; t < MTX; ++t) {
-            int row = v[t * 16];
+            for (int i = 0; i < 32; ++i) asm volatile("" : "+s"(v[i]));  // not folded into a per-lane load
 #pragma unroll
-            for (int i = 1; i < 16; ++i) row = rr == i ? v[t * 16 + i] : row;
-            aoff[t] = (static_cast<int64_t>(row / A.topk) * A.H + ch * 8) * 2;
+            for (int t = 0; t < 2; ++t) {
+                int row = v[t * 16];
+#pragma unroll
+                for (int i = 1; i < 16; ++i) row = rr == i ? v[t * 16 + i] : row;
+                aoff[h + t] = (static_cast<int64_t>(row / A.topk) * A.H + ch * 8) * 2;
+            }
         }
     };
     auto issue_w = [&](int g, int slot) {
@@ -744,7 +805,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
         for (int g = 0; g < R - 1; ++g) issue_w(g, g);
     const ConstI32* offs = as_scalar_i32(A.offsets);  // scalar loads, as above
     const int start0 = offs[e0];
-    GuPass p{0, 0, start0, offs[e0 + 1] - start0};
+    GuPass p{0, 0, start0, min(offs[e0 + 1] - start0, F::kCap)};
     const bool first_rows = p.M > 0;
     if (first_rows) {
         set_rows_first(p);
@@ -755,7 +816,7 @@ __device__ __forceinline__ void gu_flow_produce(const GuArgs& A, char* __restric
     }
     vm_wait<0>();
     dma_barrier();
-    const int4 tab = gu_flow_table(info, K);
+    const int4 tab = gu_flow_table<MTX>(info, K);
     const int S_total = gu_flow_npass<F::kPass>(K, tab) * G;  // group steps of all passes
     if (!first_rows && S_total > 0) {
         p = gu_flow_seek(0, 0, K, tab);
@@ -856,7 +917,7 @@ __device__ __forceinline__ void gu_flow_consume_pass(const GuArgs& A, char* __re
 
 template <int ACT, int NC, int MTX>
 __device__ __forceinline__ void gu_flow_consume(const GuArgs& A, char* __restrict__ lds, int w, int W, int items,
-                                                int K, bool pair) {
+                                                int K, bool pair, int E, int limit) {
     using S = GuShape<NC, 1, kFlowR>;
     using F = GuFlowShape<NC, MTX>;
     const int G = A.H >> 7;
@@ -872,11 +933,19 @@ __device__ __forceinline__ void gu_flow_consume(const GuArgs& A, char* __restric
     {
         GuSzFetch<NC, MTX> f;
         f.issue(A, e0, (t0 - e0 * nb) * S::kCols, G);
-        if (wave_id() == 0) gu_flow_fill_table(A, info, w, W, items, K, nb, S::kCols, pair);
+        // (two waves: their routing loads and scans overlap)
+        if (wave_id() < (MTX == 4 ? 2 : 1)) {
+            int cap = F::kCap;
+            // whole experts instead of chunks where the table could not hold them
+            // (the row count behind the launch's choice is the caller's word)
+            if constexpr (MTX == 4) cap = as_scalar_i32(A.offsets)[E] < limit ? F::kPass : 0x7fffffff;
+            if (wave_id() == 0) gu_flow_fill_table(A, info, w, W, items, K, nb, S::kCols, pair, cap);
+            else if constexpr (MTX == 4) gu_flow_add_chunks(A, info, w, W, E, K, nb, S::kCols, cap);
+        }
         f.commit(sz0, G);
     }
     __syncthreads();  // first barrier: the table, buffer 0 and the first pass's group 0 are ready
-    const int4 tab = gu_flow_table(info, K);
+    const int4 tab = gu_flow_table<MTX>(info, K);
     const int npass = gu_flow_npass<F::kPass>(K, tab);
     GuPass p = gu_flow_seek(0, 0, K, tab);
     const bool first_rows = __builtin_amdgcn_readlane(tab.y, 0) > 0;
@@ -917,7 +986,7 @@ __device__ __forceinline__ void gu_flow_consume(const GuArgs& A, char* __restric
 }
 
 template <int ACT, int NC, int MTX>
-__device__ __forceinline__ void gu_flow(const GuArgs& A, int W, int items, int pair) {
+__device__ __forceinline__ void gu_flow(const GuArgs& A, int W, int items, int pair, int E, int limit) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int w = blockIdx.x;
     const int K = (items - w + W - 1) / W;  // items of this workgroup (1 .. kFlowMaxItems)
@@ -926,19 +995,21 @@ __device__ __forceinline__ void gu_flow(const GuArgs& A, int W, int items, int p
         __builtin_amdgcn_s_setprio(3);
         gu_flow_produce<NC, MTX>(A, lds, w, items, K);
     } else {
-        gu_flow_consume<ACT, NC, MTX>(A, lds, w, W, items, K, pair != 0);
+        gu_flow_consume<ACT, NC, MTX>(A, lds, w, W, items, K, pair != 0, E, limit);
     }
 }
 
 template <int ACT, int NC>
 __global__ __launch_bounds__((NC + 1) * kWave) void gateup_flow_kernel(GuArgs A, int W, int items, int pair) {
-    gu_flow<ACT, NC, 2>(A, W, items, pair);
+    gu_flow<ACT, NC, 2>(A, W, items, pair, 0, 0);
 }
 
-// The wide form: passes of up to 64 rows.
+// The wide form: passes of up to 64 rows, chunks of E experts. limit: rows from
+// which the item table might not hold all chunks.
 template <int ACT, int NC>
-__global__ __launch_bounds__((NC + 1) * kWave) void gateup_flow_wide_kernel(GuArgs A, int W, int items, int pair) {
-    gu_flow<ACT, NC, 4>(A, W, items, pair);
+__global__ __launch_bounds__((NC + 1) * kWave) void gateup_flow_wide_kernel(GuArgs A, int W, int items, int pair, int E,
+                                                                            int limit) {
+    gu_flow<ACT, NC, 4>(A, W, items, pair, E, limit);
 }
 
 // Dynamic LDS beyond 64 KB: raise a kernel's limit (called once per kernel).
@@ -1005,10 +1076,17 @@ int launch_gateup_flow(const GuArgs& A, int act, int W, int items, hipStream_t s
     const int pair = items == 2 * W && (W / kXcds) % nb == 0 && (items / kXcds) % nb == 0 && W / nb <= kWave;
     auto go = [&](auto act_c) {
         constexpr int ACT = decltype(act_c)::value;
-        constexpr auto kernel = MTX == 2 ? &gateup_flow_kernel<ACT, NC> : &gateup_flow_wide_kernel<ACT, NC>;
-        static const bool attr_set = set_max_lds(reinterpret_cast<const void*>(kernel));
-        (void)attr_set;
-        hipLaunchKernelGGL(kernel, dim3(W), dim3(kThreads), lds, st, A, W, items, pair);
+        if constexpr (MTX == 2) {
+            static const bool attr_set = set_max_lds(reinterpret_cast<const void*>(&gateup_flow_kernel<ACT, NC>));
+            (void)attr_set;
+            hipLaunchKernelGGL((gateup_flow_kernel<ACT, NC>), dim3(W), dim3(kThreads), lds, st, A, W, items, pair);
+        } else {
+            static const bool attr_set = set_max_lds(reinterpret_cast<const void*>(&gateup_flow_wide_kernel<ACT, NC>));
+            (void)attr_set;
+            const int room = (kFlowMaxItems - 1 - (items + W - 1) / W) * (W / kXcds) / nb;  // chunks per XCD
+            hipLaunchKernelGGL((gateup_flow_wide_kernel<ACT, NC>), dim3(W), dim3(kThreads), lds, st, A, W, items, pair,
+                               items / nb, (room - 1) * kXcds * F::kPass);
+        }
     };
     if (act == KSL_ACT_GELU_TANH) go(std::integral_constant<int, KSL_ACT_GELU_TANH>{});
     else if (act == KSL_ACT_SILU) go(std::integral_constant<int, KSL_ACT_SILU>{});
@@ -1281,14 +1359,12 @@ __device__ __forceinline__ void dn_stage_a(const DnArgs& A, char* a_lds, int sta
 // A chunk's M tiles (up to four) go in one pass, one instance per count: with
 // passes of two, a chunk of three or four decoded its weights twice (layer of
 // 741 tokens, 46 rows per expert: 158 -> 143 us; 170 VGPRs at I = 704).
-template <int G2, bool TAIL, int LAYOUT>
-__global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
+// rows(start, M) yields the sorted rows of the workgroup, false where it has none.
+template <int G2, bool TAIL, int LAYOUT, typename Rows>
+__device__ __forceinline__ void dn_run(const DnArgs& A, int e, int h, Rows&& rows) {
     constexpr int MTX = kDnMaxMt;
     constexpr int G = 2 * G2 + (TAIL ? 1 : 0);
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
-    const int e = bid / A.nsplit;
-    const int h = bid - e * A.nsplit;
     const int col0 = h * A.tpw * 16;
     const int ncols = A.H - col0 < A.tpw * 16 ? A.H - col0 : A.tpw * 16;
     if (ncols <= 0) return;
@@ -1312,9 +1388,8 @@ __global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
         dn_fetch<G2, TAIL, LAYOUT>(x0, A, row0 + 32 * p, ln);
         dn_fetch<G2, TAIL, LAYOUT>(x1, A, row0 + 16 * t1i, ln);
     };
-    const int start = A.offsets[e];
-    const int M = A.offsets[e + 1] - start;
-    if (M <= 0) return;
+    int start, M;
+    if (!rows(start, M)) return;
     for (int m0 = 0; m0 < M; m0 += 16 * MTX) {
         const int mrows = M - m0 < 16 * MTX ? M - m0 : 16 * MTX;
         const int mt = (mrows + 15) >> 4;
@@ -1354,15 +1429,71 @@ __global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
     }
 }
 
-template <int G2, bool TAIL>
-int launch_down_g(const DnArgs& A, unsigned grid, size_t lds, int layout, hipStream_t st) {
-    static const bool attr = set_max_lds(reinterpret_cast<const void*>(&down_kernel<G2, TAIL, kDnRef>)) &&
-                             set_max_lds(reinterpret_cast<const void*>(&down_kernel<G2, TAIL, kDnTiled>));
+template <int G2, bool TAIL, int LAYOUT>
+__global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int e = bid / A.nsplit;
+    dn_run<G2, TAIL, LAYOUT>(A, e, bid - e * A.nsplit, [&](int& start, int& M) {
+        start = A.offsets[e];
+        M = A.offsets[e + 1] - start;
+        return M > 0;
+    });
+}
+
+// The same with every 64-row chunk after an expert's first in a workgroup of
+// its own: workgroups [0, first) take the first chunks as above (no search
+// before their loads), the others find theirs from the offsets, and go on a
+// round further until none is left (the row count that sized the grid is the
+// caller's word). With one workgroup walking all chunks the launch took as
+// long as the heaviest expert.
+template <int G2, bool TAIL, int LAYOUT>
+__global__ __launch_bounds__(kDnThreads) void down_spread_kernel(DnArgs A, int first, int E) {
+    constexpr int kChunk = 16 * kDnMaxMt;
+    const bool own = static_cast<int>(blockIdx.x) < first;
+    for (int bid = blockIdx.x;; bid += gridDim.x - first) {
+        int e, h, start, M;
+        if (own) {
+            const int tile = xcd_remap(bid, first);
+            e = tile / A.nsplit;
+            h = tile - e * A.nsplit;
+            start = A.offsets[e];
+            M = min(A.offsets[e + 1] - start, kChunk);
+        } else {
+            find_row_block<1>(A.offsets, E, kChunk, bid - first, A.nsplit, e, start, M, h);
+            e = __builtin_amdgcn_readfirstlane(e);
+            h = __builtin_amdgcn_readfirstlane(h);
+            start = __builtin_amdgcn_readfirstlane(start);
+            M = __builtin_amdgcn_readfirstlane(M);
+        }
+        if (M <= 0) return;
+        dn_run<G2, TAIL, LAYOUT>(A, e, h, [&](int& s, int& m) {
+            s = start;
+            m = M;
+            return true;
+        });
+        if (own) return;
+    }
+}
+
+template <int G2, bool TAIL, int LAYOUT>
+void launch_down_gl(const DnArgs& A, int64_t E, int64_t nrows, unsigned grid, size_t lds, hipStream_t st) {
+    static const bool attr = set_max_lds(reinterpret_cast<const void*>(&down_kernel<G2, TAIL, LAYOUT>)) &&
+                             set_max_lds(reinterpret_cast<const void*>(&down_spread_kernel<G2, TAIL, LAYOUT>));
     (void)attr;
-    if (layout == kDnTiled)
-        hipLaunchKernelGGL((down_kernel<G2, TAIL, kDnTiled>), dim3(grid), dim3(kDnThreads), lds, st, A);
+    // up to 512 rows (64 tokens of top-8) an expert hardly has a second chunk;
+    // else there are at most nrows / 64 chunks after the first ones
+    const unsigned more = static_cast<unsigned>((nrows / (16 * kDnMaxMt) + kXcds - 1) / kXcds * kXcds);  // >= 8
+    if (nrows <= 512)
+        hipLaunchKernelGGL((down_kernel<G2, TAIL, LAYOUT>), dim3(grid), dim3(kDnThreads), lds, st, A);
     else
-        hipLaunchKernelGGL((down_kernel<G2, TAIL, kDnRef>), dim3(grid), dim3(kDnThreads), lds, st, A);
+        hipLaunchKernelGGL((down_spread_kernel<G2, TAIL, LAYOUT>), dim3(grid + more * A.nsplit), dim3(kDnThreads), lds,
+                           st, A, static_cast<int>(grid), static_cast<int>(E));
+}
+
+template <int G2, bool TAIL>
+int launch_down_g(const DnArgs& A, int64_t E, int64_t nrows, unsigned grid, size_t lds, int layout, hipStream_t st) {
+    if (layout == kDnTiled) launch_down_gl<G2, TAIL, kDnTiled>(A, E, nrows, grid, lds, st);
+    else launch_down_gl<G2, TAIL, kDnRef>(A, E, nrows, grid, lds, st);
     KSL_LAUNCH_CHECK();
     return KSL_OK;
 }
@@ -1524,14 +1655,19 @@ int launch_gateup(const void* a16, const int32_t* sorted_rows, const int32_t* of
         // flowing across its items
         const int64_t items = E * (I / 176);
         const int W = gateup_flow_workgroups(items, H, device_cus());
-        // 64-row passes from an average of 16 rows per expert: below it hardly
-        // an expert has more than 32 rows and the forms take the same time
-        // (layer of 128 tokens 92.5 against 92.3 us, 256 tokens 99.5 / 99.0),
-        // above it the narrow form streams and decodes weights twice
-        // (layer of 384 tokens 130 -> 122 us, of 741 tokens 184 -> 157 us)
+        // 64-row chunks spread over the workgroups from more than 16 rows per
+        // expert on. At 16 (256 tokens of top-8 on 128 experts) an even routing
+        // has no second chunk and the narrow form is 2% faster (layer 97.4
+        // against 99.5 us); above it the narrow form streams and decodes weights
+        // twice (384 tokens 130 -> 116 us, 741: 184 -> 145), and with one expert's
+        // chunks in one workgroup a launch takes as long as the heaviest expert
+        // (512 tokens at popularity rank^-0.6 542 -> 180 us, 1024 tokens at
+        // rank^-1.1 1354 -> 250, both GEMMs spread).
         if (W > 0) {
-            const bool wide =
-                nrows_hint >= 16 * E && GuFlowShape<11, 4>::lds_bytes(static_cast<int>(H / 128)) <= kLdsDynMax;
+            // room in the item table for 8 chunks per XCD at least
+            const int64_t room = (kFlowMaxItems - 1 - (items + W - 1) / W) * (W / kXcds) / (I / 176);
+            const bool wide = nrows_hint > 16 * E && room >= 2 &&
+                              GuFlowShape<11, 4>::lds_bytes(static_cast<int>(H / 128)) <= kLdsDynMax;
             return wide ? launch_gateup_flow<11, 4>(A, act, W, static_cast<int>(items), st)
                         : launch_gateup_flow<11, 2>(A, act, W, static_cast<int>(items), st);
         }
@@ -1589,11 +1725,11 @@ int launch_down(const void* out2, const int32_t* offsets, const uint8_t* dn_q, c
     A.tpw = static_cast<int>(plan.tpw);
     A.nsplit = static_cast<int>(plan.nsplit);
     const int64_t grid = E * plan.nsplit;
-    if (grid >= (int64_t(1) << 31)) return KSL_ERR_SHAPE;
+    if (grid >= (int64_t(1) << 31) - 256 * plan.nsplit) return KSL_ERR_SHAPE;
     const size_t lds = plan.lds;
     switch (G) {
 #define KSL_DN_CASE(GG) \
-    case GG: return launch_down_g<GG / 2, (GG % 2) != 0>(A, static_cast<unsigned>(grid), lds, layout, st);
+    case GG: return launch_down_g<GG / 2, (GG % 2) != 0>(A, E, nrows, static_cast<unsigned>(grid), lds, layout, st);
         KSL_DN_CASE(1) KSL_DN_CASE(2) KSL_DN_CASE(3) KSL_DN_CASE(4) KSL_DN_CASE(5) KSL_DN_CASE(6)
         KSL_DN_CASE(7) KSL_DN_CASE(8) KSL_DN_CASE(9) KSL_DN_CASE(10) KSL_DN_CASE(11) KSL_DN_CASE(12)
         KSL_DN_CASE(13) KSL_DN_CASE(14) KSL_DN_CASE(15) KSL_DN_CASE(16)

@@ -698,7 +698,7 @@ def _rows_per_expert_routing(counts, topk, seed):
     # one workgroup per CU over 640 items, 64-row passes: every tile count and its edges, empty and heavy experts
     (160, 1024, 704, [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 80, 97, 128, 129, 200, 3] + [20] * 140),
     (128, 2816, 704, [33, 48, 49, 64, 65, 0, 112, 113] + [17] * 119 + [21]),  # balanced pairs
-    (128, 2816, 704, [1500] + [4] * 127),                                     # one expert holds most rows
+    (128, 2816, 704, [1500] + [5] * 127),                                     # one expert holds most rows
 ])
 def test_rows_do_not_depend_on_the_rows_beside_them(gpu, act, E, H, I, counts):
     """A token's output in a routing of many rows per expert (64-row passes,
@@ -711,7 +711,7 @@ def test_rows_do_not_depend_on_the_rows_beside_them(gpu, act, E, H, I, counts):
     counts[-1] += -sum(counts) % topk
     ids = _rows_per_expert_routing(counts, topk, E + H)
     T = ids.shape[0]
-    assert 16 * E <= T * topk <= 8192 or max(counts) > 1000
+    assert 512 < T * topk <= 8192
     w = torch.rand(T, topk, generator=torch.Generator().manual_seed(1)) + 0.1
     exp = wl.make_experts(E, H, I, 11, act=act).to(gpu)
     v2.enable_tiled_down(exp)
