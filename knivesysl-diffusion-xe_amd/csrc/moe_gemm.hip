@@ -34,7 +34,9 @@
 // to its expert (sorted slots offsets[e] .. offsets[e+1]) in chunks of up to 32
 // rows for gate/up (one or two 16-row M tiles) and 64 rows for down; with more
 // gate/up items than CUs, one persistent gate/up workgroup per CU walks
-// several of them through one LDS ring (gateup_flow_kernel). Above 8192
+// several of them through one LDS ring (gateup_flow_kernel). An expert's
+// further 64-row chunks go to other workgroups from more than 16 rows per
+// expert (gate/up, gateup_flow_wide_kernel) or 512 rows (down). Above 8192
 // routed rows both GEMMs run the GEMM-form row-block kernels of
 // moe_rbgemm.hip instead. Workgroups are remapped so that all column blocks
 // of an expert run on the same XCD (shared L2 for its activations).
