@@ -194,13 +194,13 @@ __device__ __forceinline__ void take_entropy(SmpState& st, const float (&x)[kCol
         s += e;
         t = __builtin_fmaf(d, e, t);
     }
-    if (!(t == t)) {  // a NaN, or -inf * 0, among them
+    if (!(t == t)) {  // a NaN, or -inf * 0, among them: -inf, or a finite x so far below that d overflows
         s = s0;
         t = t0;
 #pragma unroll
         for (int i = 0; i < kCols; ++i) {
-            if (!(x[i] > -INFINITY)) continue;
             const float d = x[i] - ref;
+            if (!(x[i] > -INFINITY) || d == -INFINITY) continue;  // (of x = inf d is NaN, and stays)
             const float e = __builtin_amdgcn_exp2f(d * kLog2e);
             s += e;
             t = __builtin_fmaf(d, e, t);

@@ -130,6 +130,31 @@ def test_sampler_at_the_edges_of_a_pass(gpu, V, dtype):
         assert sy[3] == ref_s[0] and ay[3] == ref_a[0]
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("top", [None, 1e32, 1e38])
+def test_entropy_of_finite_rows_wider_than_the_format(gpu, dtype, top):
+    """Finite logits whose distance from the row's maximum overflows fp32: such a
+    column has no weight, and the entropy is that of the others."""
+    ops = load_mod("fused_sampler_ops")
+    low, top = torch.finfo(dtype).min, torch.finfo(dtype).max if top is None else top
+    V = 40001
+    x = _logits(6, V, 5, dtype=dtype)
+    x[0], x[0, V // 2] = low, top               # decided: 0
+    x[1, :7], x[1, 9] = low, top
+    x[2], x[2, 0], x[2, V - 1] = low, top, top  # two equal maxima: log 2
+    x[3, ::3], x[3, 1::3], x[3, 2] = low, -float("inf"), top
+    x[4, 16384:], x[4, 0], x[4, 20000] = low, 0.0, top  # the maximum after finite passes
+    x[5, 0], x[5, 1] = low, float("inf")        # an infinite logit stays undefined
+    print(f"entropy wide rows {dtype} {top}", flush=True)
+    h = ops.fused_entropy(x.to(gpu)).cpu()
+    s, a, h2 = (t.cpu() for t in ops.sample_step(x.to(gpu), 11))
+    want = torch.tensor([0.0, 0.0, float(np.log(2.0)), 0.0, 0.0])
+    assert torch.equal(h[:5], h2[:5]) and torch.isnan(h[5]) and torch.isnan(h2[5])
+    assert (h[:5] - want).abs().max() <= 1e-6, h
+    first = torch.tensor([V // 2, 9, 0, 2, 20000, 1])
+    assert torch.equal(a, first) and torch.equal(s[[0, 1, 3, 4, 5]], first[[0, 1, 3, 4, 5]])
+
+
 def test_sampler_strided_rows_and_shapes(gpu):
     ops = load_mod("fused_sampler_ops")
     x = _logits(2 * 12, 3000, 21).reshape(2, 12, 3000)
