@@ -18,10 +18,11 @@ from . import _lib
 
 def fused_rmsnorm(x: torch.Tensor, weight: torch.Tensor | None, eps: float) -> torch.Tensor:
     # At a few hundred rows the launch costs more host time than the kernel runs:
-    # whatever is already a contiguous matrix or vector goes in as it is.
+    # whatever is already a contiguous matrix or vector goes in as it is. (A
+    # single row counts as contiguous with any stride: reshape gives it its own.)
     orig = x.shape
     flat = len(orig) == 2 and orig[1] > 0
-    x2 = x if flat and x.is_contiguous() else x.reshape(-1, orig[-1]).contiguous()
+    x2 = x if flat and orig[0] != 1 and x.is_contiguous() else x.reshape(-1, orig[-1]).contiguous()
     rows, n_cols = x2.shape
     y = torch.empty_like(x2)
     if weight is not None:

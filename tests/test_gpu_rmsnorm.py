@@ -94,6 +94,23 @@ def test_rmsnorm_empty_and_noncontiguous(gpu):
     assert torch.equal(y2, y3)
 
 
+@pytest.mark.parametrize("stride", [0, 1, 3, 8, 4096])
+def test_rmsnorm_one_row_of_any_stride(gpu, stride):
+    """A single row's stride means nothing (a window of unfold, a transposed
+    column, an expanded row): the values and a row-major result, as of the same
+    row held densely."""
+    frm = load_mod("fused_rmsnorm")
+    base = torch.randn(2816, generator=torch.Generator().manual_seed(10)).to(torch.bfloat16).to(gpu)
+    w = torch.ones(2816, dtype=torch.bfloat16, device=gpu)
+    x = base.as_strided((1, 2816), (stride, 1))
+    y = frm.fused_rmsnorm(x, w, 1e-6)
+    assert y.shape == x.shape and y.stride() == (2816, 1)
+    assert torch.equal(y, frm.fused_rmsnorm(base[None].clone(), w, 1e-6))
+    for v in (base.unsqueeze(1).t(), base.unfold(0, 2816, 5)):
+        z = frm.fused_rmsnorm(v, w, 1e-6)
+        assert z.stride() == (2816, 1) and torch.equal(z, y)
+
+
 def test_rmsnorm_zero_row(gpu):
     frm = load_mod("fused_rmsnorm")
     x = torch.zeros(4, 2816, dtype=torch.bfloat16, device=gpu)
