@@ -17,7 +17,9 @@ from . import _lib
 def router_forward(self, hidden_states: torch.Tensor):
     """(router_probabilities fp32 [T, E], top_k_weights fp32 [T, k],
     top_k_index int64 [T, k]) as DiffusionGemmaTextRouter.forward returns them."""
-    x = hidden_states if hidden_states.dim() == 2 else hidden_states.reshape(-1, hidden_states.shape[-1])
+    x = hidden_states
+    if x.dim() != 2 or x.shape[0] == 1:  # (a single token's row may have any stride)
+        x = x.reshape(-1, x.shape[-1])
     if x.stride(-1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         x = x.clone(memory_format=torch.contiguous_format)  # a fresh, aligned copy
     T, H = x.shape

@@ -88,6 +88,22 @@ def test_router_ties_take_lower_ids(gpu):
     assert torch.allclose(w.cpu(), ref.expand(T, k), rtol=1e-6)
 
 
+@pytest.mark.parametrize("stride", [0, 1, 8, 2816, 4096])
+def test_router_one_token_of_any_stride(gpu, stride):
+    """The stride of a single token's row means nothing to the drop-in call."""
+    router = load_mod("router")
+    E, H, k = 128, 2816, 8
+    rt = torch.nn.Module()
+    rt.scale, proj, rt.per_expert_scale = (t.to(gpu) for t in _params(E, H, 50))
+    rt.proj = torch.nn.Module()
+    rt.proj.weight, rt.eps = proj, 1e-6
+    rt.config = type("Config", (), {"top_k_experts": k})
+    base = torch.randn(H, generator=torch.Generator().manual_seed(51)).to(torch.bfloat16).to(gpu)
+    got = router.router_forward(rt, base.as_strided((1, H), (stride, 1)))
+    want = router.router_forward(rt, base[None].clone())
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_router_drop_in_matches_stock_module(gpu):
     """router_forward bound on a stock DiffusionGemmaTextRouter (patch_routers)
     against the unpatched module run by torch on the GPU."""
