@@ -125,8 +125,9 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 # The current stream's handle without building a torch.cuda.Stream for it
-# (0.1 against 1.5 us per call).
-_current_raw_stream = torch._C._cuda_getCurrentRawStream
+# (0.1 against 1.5 us per call). A torch without GPU support has no such call:
+# there the package imports, and raw_stream refuses its CPU tensors.
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def raw_stream(t: torch.Tensor) -> int:

@@ -113,3 +113,20 @@ def test_checkpoint_meta_refuses_a_directory_without_w4_meta(tmp_path):
     (tmp_path / "w4_meta.json").write_text('[1, 2]')
     with pytest.raises(ValueError):
         lw.checkpoint_meta(tmp_path)
+
+
+def test_package_imports_where_torch_has_no_gpu_support():
+    """On a torch built without GPU support the package still imports (its CPU
+    helpers and its refusals work); only a launch fails."""
+    import os
+    import subprocess
+    import sys
+    code = ("import torch\n"
+            "for n in [n for n in dir(torch._C) if n.startswith('_cuda')]: delattr(torch._C, n)\n"
+            "from tests.conftest import load_pkg\n"
+            "lib = load_pkg()._lib\n"
+            "try:\n    lib.stream_of(torch.zeros(1))\n"
+            "except ValueError as e:\n    print('refused:', e)\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True)
+    assert res.returncode == 0 and res.stdout.startswith("refused:"), res.stderr[-2000:]
