@@ -22,7 +22,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .fused_moe_w4_v2 import _check_act, _check_weights, dn_layout, moe_workspace, pack_ptrs
+from .fused_moe_w4_v2 import _check_act, _check_weights, check_zero_points_once, dn_layout, moe_workspace, pack_ptrs
 
 
 def _rows(t: torch.Tensor, H: int) -> torch.Tensor:
@@ -67,6 +67,7 @@ def moe_block_forward(layer, residual: torch.Tensor, hidden_states_1: torch.Tens
     if not getattr(exp, "_act_checked", False) or not hasattr(exp, "_ksl_act"):
         _check_act(exp)
     _check_weights(exp, E, H, I)
+    check_zero_points_once(exp)
     pre = layer.pre_feedforward_layernorm_2
     post2 = layer.post_feedforward_layernorm_2
     post = layer.post_feedforward_layernorm

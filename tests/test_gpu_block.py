@@ -202,3 +202,17 @@ def test_patched_layer_matches_stock_forward(gpu):
     assert ours.shape == stock.shape and ours.dtype == torch.bfloat16
     assert_tail_close(bf16_bits(ours.reshape(-1, 256)), bf16_bits(stock.reshape(-1, 256)), 0.75,
                       "patched layer vs stock forward")
+
+
+def test_block_checks_the_zero_points_of_an_unseen_module(gpu):
+    """A packed module that no load-time helper saw is checked on its first
+    block forward, as the other forwards do: a zero-point outside the contract
+    (an integer in [0, 15]) is refused, not truncated."""
+    lay, hidden, pkg = _packed_layer(gpu, 40, 73)
+    mod = load_mod("moe_block")
+    lay.experts.gu_z[3, 5, 0] = 16.0
+    with torch.no_grad(), pytest.raises(ValueError, match="zero-points"):
+        mod.moe_block_forward(lay, hidden, hidden.clone())
+    lay.experts.gu_z[3, 5, 0] = 15.0
+    with torch.no_grad():
+        assert mod.moe_block_forward(lay, hidden, hidden.clone()).shape == hidden.shape
