@@ -22,7 +22,9 @@
 // was VALU-bound. Here a division is five fused steps on the group's
 // reciprocal y (one mul, two residual corrections: Markstein's division, IBM J.
 // Res. Dev. 34, 1990), which give the correctly rounded quotient while nothing
-// over- or underflows. d >= 1e-8, and a group with a magnitude of 2^60 or more
+// over- or underflows. (The theorem needs y correctly rounded; for a divisor whose
+// mantissa is all ones one Newton step does not promise that, but gfx950's estimate
+// leads there: tests/test_gpu_load.py, at every such scale's exponent.) d >= 1e-8, and a group with a magnitude of 2^60 or more
 // takes the compiler's division; below 2^-102 a residual may be inexact, but
 // then the quotient is below 2^-71 and packs as z either way. Not kept: the
 // bytes from t = fma(w, y, z) with divisions only near a tie. bf16 weights are

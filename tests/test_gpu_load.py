@@ -205,6 +205,28 @@ def test_quantize_w4_at_ties_extremes_and_byte_offsets(gpu, dtype, gs):
         assert np.array_equal(z.cpu().numpy().view(np.uint16).reshape(N, 3), rz.view(np.uint16))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+def test_quantize_w4_at_a_scale_of_ones(gpu, dtype, gs):
+    """Scales whose mantissa is all ones, (2 - 2^-23) 2^n: there a quotient from the
+    reciprocal lies a half ulp under the division's for whole and half weights,
+    which moves it onto a rounding tie. Exact: bytes are a format."""
+    w4 = load_mod("w4a16")
+    exps = range(-4, 5) if dtype == torch.float16 else range(-20, 16)
+    v = (torch.arange(2 * gs) % 60 + 1) / 2.0  # 0.5, 1 .. 30
+    v[0] = v[gs] = 30.0
+    v[1] = v[gs + 1] = 2.0 ** -19              # range 30 - 2^-19: scale 2 - 2^-23, zero 0
+    v[gs:] *= -1.0                             # and its mirror image: zero 15
+    W = torch.stack([v * 2.0 ** n for n in exps]).to(dtype)
+    g = W.float().reshape(-1, gs)
+    assert torch.all((((g.amax(-1) - g.amin(-1)) / 15.0).view(torch.int32) & 0x7FFFFF) == 0x7FFFFF)
+    print(f"quantize scale of ones {dtype} gs={gs}", flush=True)
+    q, s, z = w4.quantize_w4(W.unsqueeze(0).to(gpu), gs)
+    oq, os_, oz = mo.quantize_w4(W.float().numpy(), gs)
+    assert np.array_equal(q[0].cpu().numpy(), oq), np.argwhere(q[0].cpu().numpy() != oq)[:4]
+    assert np.array_equal(s[0].cpu().numpy(), os_) and np.array_equal(z[0].cpu().numpy(), oz)
+
+
 class _Experts(torch.nn.Module):
     """A bf16 experts module as the model holds it before packing."""
 
