@@ -36,7 +36,7 @@
 // gate/up items than CUs, one persistent gate/up workgroup per CU walks
 // several of them through one LDS ring (gateup_flow_kernel). An expert's
 // further 64-row chunks go to other workgroups from more than 16 rows per
-// expert (gate/up, gateup_flow_wide_kernel) or 512 rows (down). Above 8192
+// expert (gate/up, gateup_flow_wide_kernel) or 256 rows (down). Above 8192
 // routed rows both GEMMs run the GEMM-form row-block kernels of
 // moe_rbgemm.hip instead. Workgroups are remapped so that all column blocks
 // of an expert run on the same XCD (shared L2 for its activations).
@@ -1358,11 +1358,15 @@ __device__ __forceinline__ void dn_stage_a(const DnArgs& A, char* a_lds, int sta
 // by the other waves of the SIMD rather than by a second register buffer (a
 // second buffer, measured, was not faster: the decode, the MFMAs with their
 // LDS reads and the stores already keep the SIMD busy while a wave waits).
-// A chunk's M tiles (up to four) go in one pass, one instance per count: with
-// passes of two, a chunk of three or four decoded its weights twice (layer of
-// 741 tokens, 46 rows per expert: 158 -> 143 us; 170 VGPRs at I = 704).
+// NTX = 4: a chunk's M tiles (up to four) go in one pass, one instance per
+// count: with passes of two, a chunk of three or four decoded its weights twice
+// (layer of 741 tokens, 46 rows per expert: 158 -> 143 us; 208 VGPRs at I = 704,
+// tiled). NTX = 2, for few rows: passes of one or two tiles, and a second pass
+// for the rare chunk of more. With the four instances in it the one-tile pass,
+// which nearly every chunk takes there, came out slower (23 tokens: 80.3 -> 81.0
+// us; with this form 80.2).
 // rows(start, M) yields the sorted rows of the workgroup, false where it has none.
-template <int G2, bool TAIL, int LAYOUT, typename Rows>
+template <int G2, bool TAIL, int LAYOUT, int NTX, typename Rows>
 __device__ __forceinline__ void dn_run(const DnArgs& A, int e, int h, Rows&& rows) {
     constexpr int MTX = kDnMaxMt;
     constexpr int G = 2 * G2 + (TAIL ? 1 : 0);
@@ -1412,7 +1416,8 @@ __device__ __forceinline__ void dn_run(const DnArgs& A, int e, int h, Rows&& row
         for (int k = 0; k < npw; ++k) {
             if (k > 0) fetch(k);
             const int p = wave + k * kDnWaves;
-            auto pass = [&](auto nt_c) {
+            // the NT M tiles whose activations start at acts, to the rows_left first rows of `to`
+            auto pass = [&](auto nt_c, const char* acts, __amdgpu_buffer_rsrc_t to, int rows_left) {
                 constexpr int NT = decltype(nt_c)::value;
                 f32x4 acc0[NT], acc1[NT];
 #pragma unroll
@@ -1420,13 +1425,25 @@ __device__ __forceinline__ void dn_run(const DnArgs& A, int e, int h, Rows&& row
                     acc0[t] = f32x4{0.f, 0.f, 0.f, 0.f};
                     acc1[t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
-                dn_pair_mma<G2, TAIL, LAYOUT, NT>(x0, x1, acc0, acc1, lds, fo, kn);
-                dn_store_pair<NT>(acc0, acc1, o_lds, out, A.H, col0 + 32 * p, 2 * p + 1 < ntiles, mrows, lane);
+                dn_pair_mma<G2, TAIL, LAYOUT, NT>(x0, x1, acc0, acc1, acts, fo, kn);
+                dn_store_pair<NT>(acc0, acc1, o_lds, to, A.H, col0 + 32 * p, 2 * p + 1 < ntiles, rows_left, lane);
             };
-            if (mt == 1) pass(std::integral_constant<int, 1>{});
-            else if (mt == 2) pass(std::integral_constant<int, 2>{});
-            else if (mt == 3) pass(std::integral_constant<int, 3>{});
-            else pass(std::integral_constant<int, 4>{});
+            if constexpr (NTX == 4) {
+                if (mt == 1) pass(std::integral_constant<int, 1>{}, lds, out, mrows);
+                else if (mt == 2) pass(std::integral_constant<int, 2>{}, lds, out, mrows);
+                else if (mt == 3) pass(std::integral_constant<int, 3>{}, lds, out, mrows);
+                else pass(std::integral_constant<int, 4>{}, lds, out, mrows);
+            } else if (mt != 1) {
+                pass(std::integral_constant<int, 2>{}, lds, out, mrows);
+                if (mt > 2) {  // of three tiles the fourth is computed from stale LDS and dropped
+                    const __amdgpu_buffer_rsrc_t rest =
+                        raw_rsrc(A.out3 + static_cast<int64_t>(start + m0 + 32) * A.H,
+                                 static_cast<uint32_t>((mrows - 32) * A.H * 2));
+                    pass(std::integral_constant<int, 2>{}, lds + 4 * G * kBlk, rest, mrows - 32);
+                }
+            } else {
+                pass(std::integral_constant<int, 1>{}, lds, out, mrows);
+            }
         }
     }
 }
@@ -1435,15 +1452,15 @@ template <int G2, bool TAIL, int LAYOUT>
 __global__ __launch_bounds__(kDnThreads) void down_kernel(DnArgs A) {
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     const int e = bid / A.nsplit;
-    dn_run<G2, TAIL, LAYOUT>(A, e, bid - e * A.nsplit, [&](int& start, int& M) {
+    dn_run<G2, TAIL, LAYOUT, 2>(A, e, bid - e * A.nsplit, [&](int& start, int& M) {
         start = A.offsets[e];
         M = A.offsets[e + 1] - start;
         return M > 0;
     });
 }
 
-// The same with every 64-row chunk after an expert's first in a workgroup of
-// its own: workgroups [0, first) take the first chunks as above (no search
+// Chunks of up to four tiles in one pass, and every 64-row chunk after an
+// expert's first in a workgroup of its own: workgroups [0, first) take the first chunks as above (no search
 // before their loads), the others find theirs from the offsets, and go on a
 // round further until none is left (the row count that sized the grid is the
 // caller's word). With one workgroup walking all chunks the launch took as
@@ -1468,7 +1485,7 @@ __global__ __launch_bounds__(kDnThreads) void down_spread_kernel(DnArgs A, int f
             M = __builtin_amdgcn_readfirstlane(M);
         }
         if (M <= 0) return;
-        dn_run<G2, TAIL, LAYOUT>(A, e, h, [&](int& s, int& m) {
+        dn_run<G2, TAIL, LAYOUT, 4>(A, e, h, [&](int& s, int& m) {
             s = start;
             m = M;
             return true;
@@ -1482,10 +1499,12 @@ void launch_down_gl(const DnArgs& A, int64_t E, int64_t nrows, unsigned grid, si
     static const bool attr = set_max_lds(reinterpret_cast<const void*>(&down_kernel<G2, TAIL, LAYOUT>)) &&
                              set_max_lds(reinterpret_cast<const void*>(&down_spread_kernel<G2, TAIL, LAYOUT>));
     (void)attr;
-    // up to 512 rows (64 tokens of top-8) an expert hardly has a second chunk;
-    // else there are at most nrows / 64 chunks after the first ones
+    // Up to 256 rows (32 tokens of top-8, an expert at most once per token) no
+    // chunk has a third tile. Above, the four-tile passes pay (61 tokens at
+    // popularity rank^-0.6 100 us in passes of two, 88 here), and there are at
+    // most nrows / 64 chunks after the first ones.
     const unsigned more = static_cast<unsigned>((nrows / (16 * kDnMaxMt) + kXcds - 1) / kXcds * kXcds);  // >= 8
-    if (nrows <= 512)
+    if (nrows <= 256)
         hipLaunchKernelGGL((down_kernel<G2, TAIL, LAYOUT>), dim3(grid), dim3(kDnThreads), lds, st, A);
     else
         hipLaunchKernelGGL((down_spread_kernel<G2, TAIL, LAYOUT>), dim3(grid + more * A.nsplit), dim3(kDnThreads), lds,

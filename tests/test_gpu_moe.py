@@ -638,6 +638,41 @@ def test_down_row_blocks_bit_equal_to_expert_mode(gpu, E, H, I, T, zipf, layout)
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("layout", ["ref", "tiled"])
+@pytest.mark.parametrize("E,H,I,counts", [
+    (16, 512, 704, [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 130, 3]),  # every tile count and its edges
+    (5, 192, 64, [33, 0, 64, 49, 97]),            # one group, column pairs that are half empty
+    (4, 256, 1024, [700, 1500, 0, 65]),           # far more chunks than a small row count plans for
+])
+def test_down_forms_agree_for_any_row_count(gpu, E, H, I, counts, layout):
+    """The down forms (passes of up to two M tiles, at most 256 rows; passes of
+    up to four with the further chunks in workgroups of their own) on the same
+    routing, and with row counts that understate it: the spare workgroups then
+    go several rounds. Same bits, and near the fp16 rounding of the float64 sums."""
+    lib, wl, v2 = load_mod("_lib"), load_mod("workloads"), load_mod("fused_moe_w4_v2")
+    nrows = sum(counts)
+    exp = wl.make_experts(E, H, I, E + I, device=gpu)
+    dn_q = v2.tiled_down(exp.dn_q, exp.dn_s, exp.dn_z) if layout == "tiled" else exp.dn_q
+    code = lib.DN_LAYOUT_TILED if layout == "tiled" else lib.DN_LAYOUT_REF
+    offsets = torch.tensor([0] + list(np.cumsum(counts)), dtype=torch.int32, device=gpu)
+    out2 = (0.5 * torch.randn(nrows, I, generator=torch.Generator().manual_seed(I))).to(torch.float16).to(gpu)
+    outs = []
+    for hint in (256, 257, 600, nrows):
+        out3 = torch.full((nrows, H), float("nan"), dtype=torch.float16, device=gpu)
+        print(f"down forms E={E} H={H} I={I} {layout} rows {nrows} hint {hint}", flush=True)
+        lib.check(lib.load().ksl_moe_down(lib.ptr(out2), lib.ptr(offsets), lib.ptr(dn_q), lib.ptr(exp.dn_s),
+                                          lib.ptr(exp.dn_z), E, H, I, hint, lib.ptr(out3), code,
+                                          lib.stream_of(out2)), "ksl_moe_down")
+        outs.append(out3)
+    torch.cuda.synchronize()
+    assert all(torch.equal(outs[0].view(torch.int16), o.view(torch.int16)) for o in outs[1:])
+    x = out2_unperm(_np(out2), I).astype(np.float64)
+    ref = np.concatenate([x[int(offsets[e]):int(offsets[e + 1])] @ mo.dequant_w4(
+        _np(exp.dn_q[e]), _np(exp.dn_s[e]), _np(exp.dn_z[e]), mo.DN_GS).astype(np.float64).T for e in range(E)])
+    check_norm_err("down", _np(outs[0]).astype(np.float32), ref.astype(np.float16).astype(np.float32),
+                   f"E={E} H={H} I={I}")  # (the bar is against the fp16 output of the exact sums)
+
+
 @pytest.mark.parametrize("E,H,I", [(128, 4096, 1024), (256, 3072, 512)])
 def test_down_at_lds_limited_shapes(gpu, E, H, I):
     """The down launch at the contract's largest shapes (I = 1024: the
