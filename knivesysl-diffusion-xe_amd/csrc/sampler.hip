@@ -3,8 +3,8 @@
 // row, one read of the row.
 //
 //   entropy: H = logsumexp(x) - sum(softmax(x) * x), online over the row
-//            (running max m, s = sum e^(x-m), t = sum x e^(x-m)); entries equal
-//            to -inf contribute nothing (torch's Categorical.entropy).
+//            (running max m, s = sum e^(x-m), t = sum (x-m) e^(x-m)); entries
+//            equal to -inf contribute nothing (torch's Categorical.entropy).
 //   sample : first index of the max of fp32(x + g), g = -log(-log(u)),
 //            u = tl.rand(seed + row, col) clamped to [1e-10, 1 - 1e-7]: Triton's
 //            generator, Philox4x32-10 on the counter (col, 0, 0, 0) with the
@@ -20,7 +20,7 @@
 //    thread draws its largest column of the first pass before anything else,
 //    which brings T near its final value at once.
 //  - The others of a wave are collected in LDS (ballot and prefix count) and
-//    drawn 64 at a time, so no lane idles in the generator.
+//    drawn 128 at a time, two per lane, so no lane idles in the generator.
 //  - For a drawn u, g = -log(-log u) <= -log(1 - u): one hardware logarithm of
 //    the generator's integer decides whether the exact score can reach T, and
 //    only then the two exact logarithms are taken (a few columns per row).
@@ -121,8 +121,7 @@ __device__ __forceinline__ T lane_tree(T v, Op op) {
         return val(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(bits(x)), decltype(ctrl)::value, 0xF, 0xF, true)));
     };
     v = op(v, move(std::integral_constant<int, 0x128>{}, v));  // row_ror:8
-    v = op(v, move(std::integral_constant<int, 0x140>{}, v));  // mirror within 16 lanes: the other half of each 8
-    v = op(v, move(std::integral_constant<int, 0x141>{}, v));  // mirror within 8
+    v = op(v, move(std::integral_constant<int, 0x140>{}, v));  // mirror within 16 lanes: lane 7 - i of each 8
     v = op(v, move(std::integral_constant<int, 0x4E>{}, v));   // quad_perm [2,3,0,1]
     return op(v, move(std::integral_constant<int, 0xB1>{}, v));
 }
@@ -194,13 +193,13 @@ __device__ __forceinline__ void take_entropy(SmpState& st, const float (&x)[kCol
         s += e;
         t = __builtin_fmaf(d, e, t);
     }
-    if (!(t == t)) {  // a NaN, or -inf * 0, among them: -inf, or a finite x so far below that d overflows
+    if (!(t == t)) {  // a NaN, or 0 * -inf: of x = -inf, or of a finite x so far below that d overflows
         s = s0;
         t = t0;
 #pragma unroll
         for (int i = 0; i < kCols; ++i) {
-            const float d = x[i] - ref;
-            if (!(x[i] > -INFINITY) || d == -INFINITY) continue;  // (of x = inf d is NaN, and stays)
+            // any of these becomes the lowest value, whose e is 0 (so does x = inf: the row ends with s = 0, a NaN)
+            const float d = fmaxf(x[i] - ref, -0x1.fffffep127f);
             const float e = __builtin_amdgcn_exp2f(d * kLog2e);
             s += e;
             t = __builtin_fmaf(d, e, t);
