@@ -18,9 +18,10 @@ It runs one wave with concrete kernel arguments and tracks:
 - every global, buffer and LDS access, checked against the buffers and LDS
   size of the launch, and whether any address, stored value or MFMA operand
   is poisoned.
-Barriers are counted, not waited on: the waves of a workgroup run one after
-another, sharing LDS (the code checked here publishes only routing scalars and
-row tables through LDS), and a test compares the waves' barrier counts."""
+run() takes one wave to its end: barriers are counted, not waited on, and a test
+compares the waves' counts. run_workgroup() takes the waves of a workgroup from
+barrier to barrier together, sharing LDS, for code that publishes a new value
+through the same LDS words in every round."""
 import re, struct, sys
 import numpy as np
 
@@ -63,6 +64,7 @@ class Wave:
         self.poison = np.zeros(256, dtype=bool)  # register may hold a stale or clobbered value
         self.spoison = [False] * 128
         self.barriers = 0  # s_barrier instructions executed (all waves of a workgroup must agree)
+        self.pc = 0  # where run() goes on, after a stop at a barrier
     # ---- operand helpers
     def sreg(self, t):
         m = re.match(r"s\[(\d+):(\d+)\]$", t)
@@ -179,8 +181,19 @@ class Wave:
 def signed32(x): return x - (1 << 32) if x & 0x80000000 else x
 def signed64(x): return x - (1 << 64) if x & (1 << 63) else x
 
-def run(ins, labels, w, max_steps=2_000_000):
-    pc = 0; steps = 0
+def run_workgroup(ins, labels, waves, max_steps=20_000_000):
+    """Take the waves (sharing one LDS) to their ends, none past a barrier that
+    another has not reached. A wave that ends early must not leave others waiting."""
+    for w in waves[1:]: w.lds = waves[0].lds
+    left = list(waves)
+    while left:
+        at = [w for w in left if run(ins, labels, w, max_steps, stop_at_barrier=True)]
+        assert not at or len(at) == len(left), "some waves ended while others wait at a barrier"
+        left = at
+
+def run(ins, labels, w, max_steps=2_000_000, stop_at_barrier=False):
+    """Run wave w to its end (False), or to its next barrier (True)."""
+    pc = w.pc; steps = 0
     U64 = np.uint64
     while True:
         steps += 1
@@ -189,7 +202,7 @@ def run(ins, labels, w, max_steps=2_000_000):
         parts = s.split(None, 1); op = parts[0]; args = parts[1] if len(parts) > 1 else ""
         t = [x for x in re.split(r",\s*|\s+", args) if x]
         pc += 1
-        if op == "s_endpgm": return
+        if op == "s_endpgm": return False
         if op.startswith("s_waitcnt"):
             m = re.search(r"vmcnt\((\d+)\)", args)
             if m:
@@ -201,7 +214,9 @@ def run(ins, labels, w, max_steps=2_000_000):
                         if r in written and len(w.trace) < 8: w.trace.append(("CLOBBER at wait", w.cur, r))
             continue
         if op == "s_barrier":
-            w.barriers += 1; continue
+            w.barriers += 1
+            if stop_at_barrier: w.pc = pc; return True
+            continue
         if op in ("s_nop", "s_setprio", "s_sleep") : continue
         if op == "s_branch": pc = labels[t[0]]; continue
         if op.startswith("s_cbranch"):

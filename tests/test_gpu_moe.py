@@ -673,6 +673,35 @@ def test_down_forms_agree_for_any_row_count(gpu, E, H, I, counts, layout):
                    f"E={E} H={H} I={I}")  # (the bar is against the fp16 output of the exact sums)
 
 
+@pytest.mark.parametrize("act", ["silu", "none"])
+@pytest.mark.parametrize("E,H,I,T,hints", [
+    (128, 1024, 704, 700, (256, 257, 700)),  # narrow (16 rows per expert), wide understated, wide
+    (9, 1024, 11264, 1600, (18, 25)),        # the item tables nearly full of chunks
+    (9, 1024, 11264, 1900, (18, 25)),        # more rows than the tables could hold: whole experts
+])
+def test_gateup_forms_agree_for_any_row_count(gpu, E, H, I, T, hints, act):
+    """The persistent gate/up forms (32-row passes; 64-row passes with the further
+    chunks in other workgroups) on the same skewed routing, also with token
+    counts that understate it: the same bits."""
+    lib, wl = load_mod("_lib"), load_mod("workloads")
+    tk = 8
+    ids, _ = wl.make_routing(T, E, tk, E + T, 1.1)
+    exp = wl.make_experts(E, H, I, E + I, device=gpu)
+    sr, off, _, a16 = _route(gpu, ids.to(gpu), wl.make_hidden(T, H, 3).to(gpu), E)
+    outs = []
+    for t_hint in hints:
+        print(f"gate/up forms E={E} H={H} I={I} T={T} {act} hint {t_hint}", flush=True)
+        out2 = torch.zeros(T * tk, 2 * I if act == "none" else I, dtype=torch.float16, device=gpu)
+        lib.check(lib.load().ksl_moe_gateup_act(lib.ptr(a16), lib.ptr(sr), lib.ptr(off), t_hint, tk, lib.ptr(exp.gu_q),
+                                                lib.ptr(exp.gu_s), lib.ptr(exp.gu_z), E, H, I,
+                                                lib.ACT_NONE if act == "none" else lib.ACT_SILU, lib.ptr(out2),
+                                                lib.stream_of(a16)), "ksl_moe_gateup_act")
+        outs.append(out2)
+    torch.cuda.synchronize()
+    assert outs[0].count_nonzero() > 0
+    assert all(torch.equal(outs[0].view(torch.int16), o.view(torch.int16)) for o in outs[1:])
+
+
 @pytest.mark.parametrize("E,H,I", [(128, 4096, 1024), (256, 3072, 512)])
 def test_down_at_lds_limited_shapes(gpu, E, H, I):
     """The down launch at the contract's largest shapes (I = 1024: the
