@@ -34,9 +34,10 @@
 // to its expert (sorted slots offsets[e] .. offsets[e+1]) in chunks of up to 32
 // rows for gate/up (one or two 16-row M tiles) and 64 rows for down; with more
 // gate/up items than CUs, one persistent gate/up workgroup per CU walks
-// several of them through one LDS ring (gateup_flow_kernel). An expert's
-// further 64-row chunks go to other workgroups from more than 16 rows per
-// expert (gate/up, gateup_flow_wide_kernel) or 256 rows (down). Above 8192
+// several of them through one LDS ring (gateup_flow_kernel; I a multiple of 176,
+// 1024 <= H <= 3072). An expert's further 64-row chunks go to other workgroups:
+// of that gate/up form from more than 16 rows per expert on
+// (gateup_flow_wide_kernel), of down above 256 rows. Above 8192
 // routed rows both GEMMs run the GEMM-form row-block kernels of
 // moe_rbgemm.hip instead. Workgroups are remapped so that all column blocks
 // of an expert run on the same XCD (shared L2 for its activations).
@@ -93,9 +94,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 constexpr int kMaxMt = 2;                        // 16-row M tiles per row chunk
 
 constexpr size_t kLdsBytes = 160 * 1024;         // LDS per workgroup on gfx950
-// Static LDS reserved beside the dynamic LDS of a launch (these kernels
-// declare none today; the reserve keeps a helper with a small __shared__
-// array from pushing a launch sized to the limit over it).
+// Static LDS reserved beside the dynamic LDS of a launch (down_spread_kernel
+// declares find_row_block's 16 bytes; the reserve keeps a helper with a small
+// __shared__ array from pushing a launch sized to the limit over it).
 constexpr size_t kLdsStatic = 64;
 constexpr size_t kLdsDynMax = kLdsBytes - kLdsStatic;
 constexpr int kGuMaxG = 32;                      // H <= 4096
@@ -632,7 +633,7 @@ __device__ __forceinline__ void gu_flow_add_chunks(const GuArgs& A, int4* __rest
     if (lane == 0) info[kFlowMaxItems - 1] = int4{n, 0, 0, 0};
 }
 
-// A pass: rows start + m0 .. start + min(M, m0 + 32) - 1 of item k (k == K: none left).
+// A pass: rows start + m0 .. start + min(M, m0 + kPass) - 1 of item k (k == K: none left).
 struct GuPass {
     int k, m0, start, M;
 };
@@ -1163,7 +1164,6 @@ struct DnArgs {
     f16* out3;
     const uint32_t* sz;     // tiled layout: the (scale, zero) pair table after the tiled weights
     int H, I, nsplit, tpw;  // tpw: 16-column tiles per workgroup
-    int early;              // weights of the first pair are requested before the routing is read
 };
 
 // LDS: activation blocks [kDnMaxMt][2G] (1 KB each, frag_pos order), then
@@ -1256,7 +1256,7 @@ __device__ __forceinline__ void dn_fetch(DnTile<G2, TAIL, LAYOUT>& w, const DnAr
 }
 
 // Both tiles of a pair against two M tiles of activations: every activation
-// fragment read from LDS feeds one MFMA of each tile. NT M tiles (1 or 2) per
+// fragment read from LDS feeds one MFMA of each tile. NT M tiles (1 to 4) per
 // pass.
 template <int G2, bool TAIL, int LAYOUT, int NT>
 __device__ __forceinline__ void dn_pair_mma(const DnTile<G2, TAIL, LAYOUT>& w0, const DnTile<G2, TAIL, LAYOUT>& w1,
@@ -1685,7 +1685,7 @@ int launch_gateup(const void* a16, const int32_t* sorted_rows, const int32_t* of
         // (512 tokens at popularity rank^-0.6 542 -> 180 us, 1024 tokens at
         // rank^-1.1 1354 -> 250, both GEMMs spread).
         if (W > 0) {
-            // room in the item table for 8 chunks per XCD at least
+            // chunks per XCD that every item table has room for (two: 512 rows)
             const int64_t room = (kFlowMaxItems - 1 - (items + W - 1) / W) * (W / kXcds) / (I / 176);
             const bool wide = nrows_hint > 16 * E && room >= 2 &&
                               GuFlowShape<11, 4>::lds_bytes(static_cast<int>(H / 128)) <= kLdsDynMax;
@@ -1734,7 +1734,6 @@ int launch_down(const void* out2, const int32_t* offsets, const uint8_t* dn_q, c
     A.out3 = static_cast<f16*>(out3);
     A.H = static_cast<int>(H);
     A.I = static_cast<int>(I);
-    A.early = nrows >= E ? 1 : 0;
     A.sz = layout == kDnTiled ? reinterpret_cast<const uint32_t*>(dn_q + E * H * (I / 2)) : nullptr;
     // large routings: the GEMM-form row-block kernel (128-row blocks)
     if (nrows > kRowBlockFrom) {

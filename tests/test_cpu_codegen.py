@@ -159,11 +159,9 @@ def test_down_kernel_addresses_and_register_flow(down_asm, E, H, I, T, tk, routi
     p_out3 = alloc("out3", nrows * H * 2)
     p_karg = alloc("kernarg", 352)
     p_sz = p_q + E * H * I // 2 if layout == 1 else 0
-    early = 1 if nrows >= E else 0
-    # DnArgs (80 bytes), down_spread_kernel's two, then the first hidden argument
+    # DnArgs (72 bytes), down_spread_kernel's two, then the first hidden argument
     # (the grid's block count)
-    karg = struct.pack("<QQQQQQQiiiii", p_out2, p_off, p_q, p_s, p_z, p_out3, p_sz, H, I, nsplit, tpw, early)
-    karg += b"\0" * (80 - len(karg))
+    karg = struct.pack("<QQQQQQQiiii", p_out2, p_off, p_q, p_s, p_z, p_out3, p_sz, H, I, nsplit, tpw)
     karg += (struct.pack("<ii", first, E) if spread else b"") + struct.pack("<I", grid) + b"\0" * 60
     mem = {p_karg + k: struct.unpack("<I", karg[k:k + 4])[0] for k in range(0, len(karg), 4)}
     mem.update({p_off + 4 * e: int(offsets[e]) for e in range(E + 1)})
