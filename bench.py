@@ -115,10 +115,12 @@ def stage_bytes(n_touched: int) -> dict:
             "ffn": gu + dn - T * TOPK * I * 2, "combine": combine_algorithmic_bytes()}
 
 
-# rocprofv3 kernel names of the stages (substring match on the demangled name)
+# rocprofv3 kernel names of the stages (substrings of the name; down runs
+# down_kernel or down_spread_kernel by the number of rows)
 LATENCY_STAGES = ("route_norm", "combine")  # timed by graph replay (see pass 2)
-STAGE_KERNELS = {"route_norm": "route", "gateup": "gateup_", "down": "down_kernel",
-                 "ffn": "ffn_kernel", "combine": "combine_kernel"}
+STAGE_KERNELS = {"route_norm": ("route",), "gateup": ("gateup_",),
+                 "down": ("::down_kernel", "11down_kernel", "down_spread_kernel"),
+                 "ffn": ("ffn_kernel",), "combine": ("combine_kernel",)}
 
 
 def summarize_pmc(fetch_dir: str, write_dir: str) -> int:
@@ -152,10 +154,13 @@ def summarize_pmc(fetch_dir: str, write_dir: str) -> int:
     fr, wr = copy_factor(fd), copy_factor(wd)
     out = {"source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE over bench.py --copy-calibration",
            "unit": "bytes per dispatch", "fetch_scale": fr, "write_scale": wr, "kernels": {}}
-    for stage, key in STAGE_KERNELS.items():
-        names = [k for k in fetch if key in k]
-        if not names:
+    ffn = any("ffn_kernel" in k for k in fetch)
+    for stage, keys in STAGE_KERNELS.items():
+        if stage in (("gateup", "down") if ffn else ("ffn",)):
             continue
+        names = [k for k in fetch if any(key in k for key in keys)]
+        if not names:
+            raise SystemExit(f"no kernel of the {stage} stage among {sorted(fetch)}")
         name = max(names, key=lambda k: fetch[k][1])
         f_kib, n = fetch[name]
         w_kib = write.get(name, (0.0, 0))[0]
