@@ -17,12 +17,13 @@ from . import _lib
 def router_forward(self, hidden_states: torch.Tensor):
     """(router_probabilities fp32 [T, E], top_k_weights fp32 [T, k],
     top_k_index int64 [T, k]) as DiffusionGemmaTextRouter.forward returns them."""
-    x = hidden_states
-    if x.dim() != 2 or x.shape[0] == 1:  # (a single token's row may have any stride)
-        x = x.reshape(-1, x.shape[-1])
+    x, shape = hidden_states, hidden_states.shape
+    if len(shape) != 2 or shape[0] == 1:  # (a single token's row may have any stride)
+        x = x.reshape(-1, shape[-1])
+        shape = x.shape
     if x.stride(-1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
         x = x.clone(memory_format=torch.contiguous_format)  # a fresh, aligned copy
-    T, H = x.shape
+    T, H = shape
     proj = self.proj.weight
     E = proj.shape[0]
     k = int(self.config.top_k_experts)
